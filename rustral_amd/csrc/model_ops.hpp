@@ -1,6 +1,8 @@
-// model_ops.hpp -- internal entry of model_ops.hip shared by the decoder and
-// the serving engine.
+// model_ops.hpp -- what projection.hip, model_ops.hip, the decoder and the serving
+// engine share.
 #pragma once
+
+#include <type_traits>
 
 #include "common.hpp"
 
@@ -13,5 +15,24 @@ namespace rkv {
 int linear_launch(float* y, const float* x, const float* w, const float* b, const float* res,
                   int epi, int rows, int in_dim, int out_dim, hipStream_t s,
                   const float* ln_g = nullptr, const float* ln_b = nullptr, float eps = 0.0f);
+
+// 0.5 v (1 + tanh(sqrt(2 / pi) (v + 0.044715 v^3))), the reference's order.
+__device__ __forceinline__ float gelu_f(float v) {
+#pragma clang fp contract(off)
+  const float k = sqrtf(2.0f / 3.14159265358979323846f);
+  const float x3 = v * v * v;
+  const float xp = v + 0.044715f * x3;
+  const float t = tanhf(k * xp);
+  return 0.5f * v * (1.0f + t);
+}
+
+// Calls f(std::integral_constant<int, I>) for I = B .. E-1 in order.
+template <int B, int E, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+  if constexpr (B < E) {
+    f(std::integral_constant<int, B>{});
+    static_for<B + 1, E>(f);
+  }
+}
 
 }  // namespace rkv

@@ -221,6 +221,38 @@ def test_gpu_linear_bit_exact(torch_dev, rows, i, o):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,i,o,skew", [
+    (1, 1, 1, 0), (2, 129, 17, 0),            # 16 columns a wave, one-wave workgroups
+    (3, 64, 16, 0), (7, 191, 200, 1),         # ... four rows a workgroup; rows not 16-byte aligned
+    (16, 1024, 1025, 0), (6, 128, 2800, 0),   # 64 columns a wave, one row each
+    (9, 63, 4111, 3), (64, 256, 2048, 0),
+    (65, 260, 2049, 0), (66, 65, 2111, 1),    # four rows a wave (matrix-core products)
+    (129, 4, 1100, 0), (61, 8192, 2200, 0)])
+def test_gpu_linear_splits_bit_exact(torch_dev, rows, i, o, skew):
+    """Every split of the projection kernel at the edges of its chunks (64
+    features, pairs of them unguarded), column groups and row groups: equal to
+    the oracle's serial sums bit for bit, with exact zeros, denormal products
+    and sums that cancel among the terms."""
+    torch, dev = torch_dev
+    rng = np.random.default_rng(rows * 1000 + i + o)
+    x = rng.standard_normal((rows, i)).astype(np.float32)
+    w = (rng.standard_normal((o, i)) * 0.05).astype(np.float32)
+    x[:, ::5] = 0.0
+    x[0, 1::7] = -0.0
+    w[::3, 2::11] = 1e-38
+    x[-1, 2::11] *= np.float32(1e-4)
+    w[::2, 3::8] *= 1e6
+
+    def t(a):  # skew floats past a 16-byte boundary
+        flat = torch.zeros(a.size + skew, device=dev)
+        flat[skew:] = torch.from_numpy(np.ascontiguousarray(a)).to(dev).reshape(-1)
+        return flat[skew:].view(a.shape)
+
+    got = model.linear(t(x), t(w)).cpu().numpy()
+    assert np.array_equal(got, oracle.linear(x, w))
+
+
+@pytest.mark.gpu
 def test_gpu_layer_norm_add_embed_bit_exact(torch_dev):
     torch, dev = torch_dev
     rng = np.random.default_rng(3)
@@ -270,6 +302,9 @@ def test_gpu_decoder_on_a_caller_stream(dev):
     (300, 128, 4, 2, "f32", True, True),      # a prompt's rows, GQA
     (7, 256, 8, 1, "bf16", True, False),
     (5, 4096, 32, 8, "bf16", False, True),    # Llama-3-8B layer shape
+    (64, 136, 4, 4, "f32", True, True),       # 64 columns a wave, one row each
+    (260, 192, 6, 2, "bf16", True, True),     # four rows a wave, an odd chunk at the end
+    (700, 72, 3, 1, "f32", False, False),     # ... without the norm
     (3, 33, 3, 1, "f32", True, True)])        # odd d_model: the scalar weight path
 def test_gpu_qkv_append_bit_exact(torch_dev, n, d, hq, hkv, dtype, ln, bias):
     """The fused LN1 -> q / k / v -> append launch equals the oracle's
