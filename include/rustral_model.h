@@ -109,9 +109,9 @@ int rkv_argmax(int32_t* out, const float* x, int rows, int n, void* stream);
  * q,k,v = h W^T + b, K/V appended to a paged fp32 pool (16-token blocks from
  * a host block manager), a = paged decode attention (rkv_decode_attention)
  * W_o^T + b_o, x += a, x += W_2 gelu(W_1 LN2(x) + b_1) + b_2; logits =
- * LN_f(x) W_lm^T; next id = argmax.  The prompt is fed one token per step
- * (equal to a causal prefill: each step attends to the cache including
- * itself).  Follows tape_transformer.rs:87-139 (per-head attention) and
+ * LN_f(x) W_lm^T; next id = argmax.  The prompt runs as rows of one pass
+ * (up to 64 positions at a time), each attending to the cache up to itself
+ * (a causal prefill).  Follows tape_transformer.rs:87-139 (per-head attention) and
  * :209-247 (pre-LN block), transformer.rs:69-82 (PE) and :789 (lm_head
  * without bias).
  *

@@ -478,6 +478,25 @@ def test_gpu_per_head_recipe_on_device_ops_matches_paged_decode(torch_dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n_prompt,n_new,max_seq", [(1, 3, 3), (63, 4, 128), (64, 4, 128),
+                                                    (65, 4, 128), (150, 2, 700)])
+def test_gpu_decoder_prompt_chunks(torch_dev, n_prompt, n_new, max_seq):
+    """Prompts around the 64 positions a pass takes, and with more than one
+    attention partition per row (max_seq 700): tokens and logits as the
+    oracle's, which feeds one position at a time."""
+    cfg = model.config(max_seq=max_seq)
+    params = model.init_params(cfg, seed=5, std=0.05)
+    prompt = np.random.default_rng(n_prompt).integers(0, 1000, n_prompt).astype(np.int32)
+    dec = model.Decoder(cfg, params)
+    want, want_lg = oracle.decoder_generate(oracle.decoder_config(max_seq=max_seq), params, prompt,
+                                            n_new, logits=True)
+    for _ in range(2):  # captured, then replayed
+        got, lg = dec.generate(prompt, n_new, logits=True)
+        assert got.tolist() == want.tolist()
+        assert np.all(np.abs(lg - want_lg) <= np.maximum(1e-4, 1e-3 * np.abs(want_lg)))
+
+
+@pytest.mark.gpu
 def test_gpu_decoder_pool_size_does_not_change_tokens(dev):
     """The same weights in decoders of max_seq 1024 and 128 (64 and 8 KV
     blocks per layer, other attention grids): tokens equal the CPU
