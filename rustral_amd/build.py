@@ -55,7 +55,7 @@ def _stale(src: str) -> bool:
     obj = _obj(src)
     if not os.path.exists(obj):
         return True
-    deps = [src, os.path.join(CSRC, "common.hpp"), os.path.join(CSRC, "model_ops.hpp"), *[
+    deps = [src, os.path.join(CSRC, "common.hpp"), *[os.path.join(CSRC, h) for h in os.listdir(CSRC) if h.endswith(".hpp")], *[
         os.path.join(HERE, "..", "include", h) for h in os.listdir(os.path.join(HERE, "..", "include"))]]
     t = os.path.getmtime(obj)
     return any(os.path.getmtime(d) > t for d in deps if os.path.exists(d))
