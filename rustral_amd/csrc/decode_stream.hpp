@@ -98,11 +98,9 @@ constexpr int split_of() { return sizeof(T) == 1 ? RKV_DECODE_SPLIT_Q : RKV_DECO
 
 // Partition sizes.  A call's partition size P (tokens) is any multiple of
 // 16 * SPLIT up to the build's largest (640); its waves stream
-// tw = P / (16 * SPLIT) tiles each.  The kernels are built for two slice
-// lengths: the largest, and for 16-bit and fp32 pools also 512 tokens, so
-// that a caller asking for 512-token partitions runs them without masked
-// slots; other sizes run on the smallest build that holds them, the extra
-// slots masked.
+// tw = P / (16 * SPLIT) tiles each.  The kernels are built for several slice
+// lengths (pick_p); a size between runs on the smallest build that holds it,
+// the extra slots masked.
 // bf16 pools also have two builds of 8-wave workgroups: 768 tokens (a
 // 96-token slice, 6 tiles, per wave) and 1280 tokens (10 tiles per wave, the
 // 640-token build's slice); requests that are multiples of 128 above 640 run
@@ -124,6 +122,11 @@ constexpr int kSmallP = 512;
 static_assert(kSmallP <= kP && kSmallP % (16 * RKV_DECODE_SPLIT) == 0, "small partition build");
 static_assert(kSmallP <= kPQ && kSmallP % (16 * RKV_DECODE_SPLIT_Q) == 0,
               "small partition build of the 1-byte pools");
+// Builds of 128, 256 and 384 tokens for contexts that short (pick_p).
+constexpr int kShortP = 128;
+static_assert(kShortP % (2 * 16 * RKV_DECODE_SPLIT) == 0 &&
+                  kShortP % (2 * 16 * RKV_DECODE_SPLIT_Q) == 0 && 3 * kShortP < kSmallP,
+              "short partition builds (1-byte V tiles go in pairs)");
 constexpr int kWideSplit = 8;
 constexpr int kWideP1 = 768, kWideP2 = 1280;
 static_assert(kWideP1 % (16 * kWideSplit) == 0 && kWideP2 % (16 * kWideSplit) == 0 &&
@@ -1236,8 +1239,16 @@ Launch make_launch(bool append) {
 }
 
 // The build for partitions of P tokens: above the largest 4-wave build (bf16
-// pools), the smallest 8-wave build that holds them; else the 512-token
-// build when it holds them, else the largest.
+// pools), the smallest 8-wave build that holds them; else the smallest 4-wave
+// build that does.  A build's slots past the partition cost almost what live
+// ones do, so short contexts have builds of their own (us per call, Llama-3-8B
+// head shape, bf16 unless noted, the 512-token build -> the smallest that
+// holds the call): 1 sequence of 100 tokens 9.5 -> 5.3, of 300 9.5 -> 8.0; 64
+// of 10 .. 120 15.6 -> 8.8, of 100 .. 250 17.1 -> 12.7, of 100 .. 380 18.8 ->
+// 16.4; 256 of 50 .. 120 47 -> 23, of 200 .. 380 67 -> 58; int8 256 of 100 ..
+// 250 30 -> 22; fp32 pools, head_dim 32, 1 of 60 .. 128 4.3 -> 2.7.  Eight
+// waves on the same tokens are slower (100 tokens 6.9 against 6.4 with 256
+// token slots), and so is a deeper ring below 200 sequences.
 template <typename T, int D, int G, int FMT>
 Launch pick_p(int P, bool append) {
   if constexpr (FMT == RKV_BF16) {
@@ -1246,6 +1257,9 @@ Launch pick_p(int P, bool append) {
       return make_launch<T, D, G, FMT, kWideP2 / kBS, kWideSplit>(append);
     }
   }
+  if (P <= kShortP) return make_launch<T, D, G, FMT, kShortP / kBS>(append);
+  if (P <= 2 * kShortP) return make_launch<T, D, G, FMT, 2 * kShortP / kBS>(append);
+  if (P <= 3 * kShortP) return make_launch<T, D, G, FMT, 3 * kShortP / kBS>(append);
   if constexpr (kSmallP < part_of<T>()) {
     if (P <= kSmallP) return make_launch<T, D, G, FMT, kSmallP / kBS>(append);
   }

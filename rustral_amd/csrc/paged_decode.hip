@@ -382,11 +382,15 @@ void split_ws(void* ws, int B, int Hq, int D, int max_parts, float*& acc, float*
 
 int launch_partitions(const DecodeArgs& a, int max_parts, int P) {
   const int G = a.num_q_heads / a.num_kv_heads;
+  const int cap = ctx_cap_of(a.max_context, a.max_blocks_per_seq, a.block_size);
+  // One partition per sequence has to hold the context cap, not P: up to 512
+  // tokens the smallest build that does (pick_p).
+  if (max_parts == 1 && cap <= kSmallP)
+    P = cap <= kShortP ? kShortP : (cap + kShortP - 1) / kShortP * kShortP;
   Launch l = pick(a.dtype, a.head_dim, G, P, a.k_new != nullptr);
   if (!l.kernel) return fail(RKV_ERR_UNSUPPORTED, "no decode kernel for this shape");
   float *acc = nullptr, *ml = nullptr;
   if (max_parts > 1) split_ws(a.workspace, a.num_seqs, a.num_q_heads, a.head_dim, max_parts, acc, ml);
-  const int cap = ctx_cap_of(a.max_context, a.max_blocks_per_seq, a.block_size);
   // KV-head major: the Hkv workgroups of one (partition, sequence) are adjacent
   const dim3 grid((unsigned)a.num_kv_heads, (unsigned)max_parts, (unsigned)a.num_seqs);
   const size_t pad = (a.dtype == RKV_BF16 && a.head_dim == 128) ? RKV_DECODE_LDS_PAD_16 : 0;

@@ -282,6 +282,28 @@ def test_decode_caller_partition_sizes(dev, dtype, P):
     assert_allclose_ref(to_np(out), want, RTOL, ATOL, f"partition {P} vs oracle")
 
 
+@pytest.mark.parametrize("cap", [16, 128, 144, 256, 272, 384, 400, 512, 528])
+@pytest.mark.parametrize("dtype,hq,hkv,d", [("f32", 4, 4, 32), ("f32", 8, 2, 128),
+                                            ("bf16", 32, 8, 128), ("bf16", 16, 2, 64),
+                                            ("bf16", 8, 8, 32)])
+def test_decode_short_context_builds(dev, cap, dtype, hq, hkv, d):
+    """Calls of one partition run on the smallest build that holds their
+    context cap (128, 256, 384, 512 tokens): caps at the builds' edges, with
+    contexts at the cap, inside its last block, at wave slices' edges, empty
+    and beyond the cap (clamped)."""
+    ctx = np.array([cap, cap - 1, cap - 15, cap // 2 + 1, 1, 0, min(cap, 33), cap], np.int32)
+    say(f"decode short cap={cap} {dtype} hq={hq} hkv={hkv} d={d}")
+    q, kp, vp, kf, vf, tables = case(cap + hq + d, len(ctx), hq, hkv, d, ctx, dtype)
+    scale = float(np.float32(1.0 / math.sqrt(d)))
+    over = ctx.copy()
+    over[-1] += 9
+    out = kv.decode_attention(to_dev(q, dev), to_dev(kp, dev), to_dev(vp, dev), to_dev(tables, dev),
+                              to_dev(over, dev), scale, max_context=cap)
+    torch.cuda.synchronize()
+    want = oracle.decode_attention(q, kp, vp, tables, ctx, scale)
+    assert_allclose_ref(to_np(out), want, RTOL, ATOL, f"context cap {cap} vs oracle")
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (16, 2, 128), (8, 8, 64), (8, 4, 32),
                                       (64, 8, 128)])
 @pytest.mark.parametrize("P", [768, 896, 1024, 1280, 0])

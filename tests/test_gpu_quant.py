@@ -180,6 +180,30 @@ def test_decode_q_matches_oracle_on_dequantized_pool(dev, fmt, hq, hkv, d):
     assert_allclose_ref(got, want, RTOL, ATOL, "gpu vs oracle (dequantized pool)")
 
 
+@pytest.mark.parametrize("cap", [16, 128, 144, 256, 272, 384, 400, 512])
+@pytest.mark.parametrize("fmt,hq,hkv,d", [("int8", 32, 8, 128), ("int8", 8, 1, 64),
+                                          ("fp8", 8, 2, 128)])
+def test_decode_q_short_context_builds(dev, cap, fmt, hq, hkv, d):
+    """1-byte pools on the builds for contexts of 128, 256, 384 and 512
+    tokens: caps at their edges, the rows past a context holding canaries."""
+    say(f"decode_q short cap={cap} fmt={fmt} hq={hq} hkv={hkv} d={d}")
+    rng = np.random.default_rng(cap + d)
+    ctx = np.array([cap, cap - 1, cap - 15, cap // 2 + 1, 1, 0, min(cap, 33)], np.int32)
+    bs = 16
+    nb = int(sum((c + bs - 1) // bs for c in ctx)) + 2
+    tables = make_tables(rng, ctx, bs, nb)
+    slots = np.concatenate([tables[b, np.arange(L) // bs].astype(np.int64) * bs + np.arange(L) % bs
+                            for b, L in enumerate(ctx)])
+    kp, vp, ks, vs = quant_case(cap + hq, nb, hkv, bs, d, fmt, fill_slots=slots)
+    q = rng.standard_normal((len(ctx), hq, d)).astype(np.float32)
+    scale = float(np.float32(1 / math.sqrt(d)))
+    got = run_q(dev, q, kp, vp, ks, vs, tables, ctx, scale, fmt, max_context=cap)
+    kf = oracle.dequantize_pool(kp, ks, CODE[fmt])
+    vf = oracle.dequantize_pool(vp, vs, CODE[fmt])
+    want = oracle.decode_attention(q, kf, vf, tables, ctx, scale)
+    assert_allclose_ref(got, want, RTOL, ATOL, f"context cap {cap} vs oracle")
+
+
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
 def test_decode_q_config2_shape_and_partial_blocks(dev, fmt):
     """configs[2] shape (B64, Hq32, Hkv8, D128, L in U[512, 4096]); only the
