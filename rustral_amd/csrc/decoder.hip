@@ -340,7 +340,8 @@ int enqueue_generation(rkv_decoder* dec, int n_prompt, int total, hipStream_t s)
   int produced = 0;
   for (int p = 0, n = 0; p < total; p += n) {  // positions p .. p + n - 1
     n = p < n_prompt ? std::min(dec->chunk, n_prompt - p) : 1;
-    RKV_TRY(rkv_embed(dec->x, P, dec->ids + p, dec->pe, dec->pos + p, n, V, d, c.max_seq, s));
+    if (p < n_prompt)  // later rows are embedded where their id is found
+      RKV_TRY(rkv_embed(dec->x, P, dec->ids + p, dec->pe, dec->pos + p, n, V, d, c.max_seq, s));
     for (int l = 0; l < c.n_layers; ++l) {
       const LayerOffsets o = layer_offsets(c, l);
       float* kp = dec->k_pool + l * layer_pool;
@@ -363,7 +364,11 @@ int enqueue_generation(rkv_decoder* dec, int n_prompt, int total, hipStream_t s)
     float* lg = dec->logits + (int64_t)produced * V;
     RKV_TRY(linear_launch(lg, dec->x + (int64_t)(n - 1) * d, P + fin + 2 * d, nullptr, nullptr, 0,
                           1, d, V, s, P + fin, P + fin + d, c.eps));
-    RKV_TRY(rkv_argmax(dec->ids + p + n, lg, 1, V, s));
+    if (p + n < total)
+      RKV_TRY(argmax_embed_launch(dec->ids + p + n, dec->x, lg, V, P,
+                                  dec->pe + (int64_t)(p + n) * d, d, s));
+    else
+      RKV_TRY(rkv_argmax(dec->ids + p + n, lg, 1, V, s));
     ++produced;
   }
   return RKV_OK;

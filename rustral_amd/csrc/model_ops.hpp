@@ -16,6 +16,11 @@ int linear_launch(float* y, const float* x, const float* w, const float* b, cons
                   int epi, int rows, int in_dim, int out_dim, hipStream_t s,
                   const float* ln_g = nullptr, const float* ln_b = nullptr, float eps = 0.0f);
 
+// rkv_argmax of one row of logits and rkv_embed of the winner (pe_row: its
+// position's row of the positional table) in one launch.
+int argmax_embed_launch(int32_t* id, float* x_next, const float* logits, int vocab,
+                        const float* table, const float* pe_row, int dim, hipStream_t s);
+
 // 0.5 v (1 + tanh(sqrt(2 / pi) (v + 0.044715 v^3))), the reference's order.
 __device__ __forceinline__ float gelu_f(float v) {
 #pragma clang fp contract(off)

@@ -44,6 +44,7 @@ struct ProjArgs {
   void *k_pool, *v_pool;
   const int64_t* slots;
   int q_dim, kvd, num_kv_heads, head_dim, block_size;
+  int hd_log2, bs_log2;  // of powers of two, else -1
   int64_t num_slots;
 };
 
@@ -58,21 +59,47 @@ __device__ __forceinline__ const float* weight_row(const ProjArgs& a, int o) {
   return w + (int64_t)o * a.n;
 }
 
-__device__ __forceinline__ void put(const ProjArgs& a, int r, int o, float sum) {
+// What put needs of column o and row r besides the sum, read before the sums
+// start so that the end of a wave does not wait for memory again.
+struct ColTail {
+  float b;     // bias (0 with has_b false)
+  bool has_b;
+};
+struct RowTail {
+  float res;     // kResidual
+  int64_t slot;  // kQkv
+};
+__device__ __forceinline__ ColTail col_tail(const ProjArgs& a, int o) {
+  const float* b = a.b;
+  if (a.mode >= kQkvF32 && o >= a.q_dim) {
+    o -= a.q_dim;
+    b = o < a.kvd ? a.bk : a.bv;
+    if (o >= a.kvd) o -= a.kvd;
+  }
+  return ColTail{b ? b[o] : 0.0f, b != nullptr};
+}
+__device__ __forceinline__ RowTail row_tail(const ProjArgs& a, int r, int o) {
+  return RowTail{a.mode == kResidual ? a.res[(int64_t)r * a.cols + o] : 0.0f,
+                 a.mode >= kQkvF32 ? a.slots[r] : 0};
+}
+
+__device__ __forceinline__ void put(const ProjArgs& a, int r, int o, float sum, const ColTail& c,
+                                    const RowTail& t) {
 #pragma clang fp contract(off)
+  const float v = c.has_b ? sum + c.b : sum;
   if (a.mode >= kQkvF32) {
     if (o < a.q_dim) {
-      a.y[(int64_t)r * a.q_dim + o] = a.b ? sum + a.b[o] : sum;
+      a.y[(int64_t)r * a.q_dim + o] = v;
       return;
     }
     const bool is_v = o >= a.q_dim + a.kvd;
     const int col = o - a.q_dim - (is_v ? a.kvd : 0);
-    const float* b = is_v ? a.bv : a.bk;
-    const float v = b ? sum + b[col] : sum;
-    const int64_t slot = a.slots[r];
+    const int64_t slot = t.slot;
     if (slot < 0 || slot >= a.num_slots) return;  // padding or out-of-range slot
-    const int64_t blk = slot / a.block_size, row = slot - blk * a.block_size;
-    const int h = col / a.head_dim, e = col - h * a.head_dim;
+    const int64_t blk = a.bs_log2 >= 0 ? slot >> a.bs_log2 : slot / a.block_size;
+    const int64_t row = slot - blk * a.block_size;
+    const int h = a.hd_log2 >= 0 ? col >> a.hd_log2 : col / a.head_dim;
+    const int e = col - h * a.head_dim;
     const int64_t dst = ((blk * a.num_kv_heads + h) * a.block_size + row) * a.head_dim + e;
     void* pool = is_v ? a.v_pool : a.k_pool;
     if (a.mode == kQkvBf16)
@@ -81,9 +108,8 @@ __device__ __forceinline__ void put(const ProjArgs& a, int r, int o, float sum) 
       static_cast<float*>(pool)[dst] = v;
     return;
   }
-  const int64_t at = (int64_t)r * a.cols + o;
-  const float v = a.b ? sum + a.b[o] : sum;
-  a.y[at] = a.mode == kResidual ? a.res[at] + v : (a.mode == kGelu ? gelu_f(v) : v);
+  a.y[(int64_t)r * a.cols + o] =
+      a.mode == kResidual ? t.res + v : (a.mode == kGelu ? gelu_f(v) : v);
 }
 
 // Elements k .. k + 3 of a row of n floats without a branch: past the row's
@@ -261,16 +287,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
     const int r = r0 + (i < RW ? i : 0);
     return a.x + (int64_t)(r < a.rows ? r : a.rows - 1) * n;
   };
-  float2 st[NX];
-  if constexpr (LN) {
-    const float2 s4 = row_stats<VEC>(row_of(lane >> 4), n, a.eps, s_buf + wave * 8 * kRow);
-#pragma unroll
-    for (int i = 0; i < NX; ++i) {
-      const int src = 16 * (MFMA ? lane & 3 : i);
-      st[i] = make_float2(__shfl(s4.x, src), __shfl(s4.y, src));
-    }
-    lds_barrier();  // the buffers become weights
-  }
   const int xk = 4 * (MFMA ? lane >> 2 : lane & 15);
   const float* xrow[NX];
 #pragma unroll
@@ -285,6 +301,27 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
       bv[p] = load4u<VEC>(a.ln_b + k);
     }
   };
+  if (pairs) {
+    xload(0, 0);
+    xload(1, 1);
+  }
+  // the output column and rows of this lane (duplicates and rows past the end
+  // clamped: loaded, not stored)
+  const int o = o0 + lane % OW, oc = o < a.cols ? o : a.cols - 1;
+  const ColTail ct = col_tail(a, oc);
+  RowTail rt[RW];
+#pragma unroll
+  for (int e = 0; e < RW; ++e) rt[e] = row_tail(a, r0 + e < a.rows ? r0 + e : a.rows - 1, oc);
+  float2 st[NX];
+  if constexpr (LN) {
+    const float2 s4 = row_stats<VEC>(row_of(lane >> 4), n, a.eps, s_buf + wave * 8 * kRow);
+#pragma unroll
+    for (int i = 0; i < NX; ++i) {
+      const int src = 16 * (MFMA ? lane & 3 : i);
+      st[i] = make_float2(__shfl(s4.x, src), __shfl(s4.y, src));
+    }
+    lds_barrier();  // the buffers become weights
+  }
   float *cur = s_buf, *next = s_buf + WB, *spare = s_buf + 2 * WB;
   const int wl = (lane % OW) * kRow;  // this lane's column in a buffer
   const f32x4_t zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -366,8 +403,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   constexpr std::true_type looped{};
   constexpr std::false_type last{};
   if (pairs) {
-    xload(0, 0);
-    xload(1, 1);
     wstore(wv[0], cur);
     wload(wv[0], 2);
     lds_barrier();
@@ -403,11 +438,10 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
       for (int e = 0; e < RW; ++e) acc[e] = acc[e] + p[1][t][e];  // a chunk has an even count
   }
 
-  const int o = o0 + lane;
   if (lane < OW && o < a.cols) {
 #pragma unroll
     for (int e = 0; e < RW; ++e)
-      if (r0 + e < a.rows) put(a, r0 + e, o, acc[e]);
+      if (r0 + e < a.rows) put(a, r0 + e, o, acc[e], ct, rt[e]);
   }
 }
 
@@ -524,6 +558,8 @@ extern "C" int rkv_qkv_append(float* q_out, void* k_pool, void* v_pool,
   a.slots = slot_mapping, a.num_slots = num_blocks * block_size;
   a.q_dim = q_dim, a.kvd = num_kv_heads * head_dim;
   a.num_kv_heads = num_kv_heads, a.head_dim = head_dim, a.block_size = block_size;
+  const auto log2_of = [](int v) { return (v & (v - 1)) == 0 ? __builtin_ctz(v) : -1; };
+  a.hd_log2 = log2_of(head_dim), a.bs_log2 = log2_of(block_size);
   a.rows = n_tokens, a.n = d_model, a.cols = q_dim + 2 * a.kvd;
   a.mode = dtype == RKV_BF16 ? kQkvBf16 : kQkvF32;
   return dispatch(a, aligned16(wq) && aligned16(wk) && aligned16(wv),
