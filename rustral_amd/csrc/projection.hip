@@ -196,9 +196,16 @@ __device__ __forceinline__ float2 row_stats(const float* xr, int n, float eps, f
         }
       }
     }
-    for (int k = full * kChunk; k < n; k += kChunk) {
-      put_chunk(0, keep4(term(load4<VEC>(xr, k + k4, n)), k + k4, n));
-      add_chunk(0);
+    f32x4_t last[4];  // the chunks past full, requested together
+#pragma unroll
+    for (int u = 0; u < 4; ++u) last[u] = load4<VEC>(xr, (full + u) * kChunk + k4, n);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = (full + u) * kChunk;
+      if (k < n) {
+        put_chunk(0, keep4(term(last[u]), k + k4, n));
+        add_chunk(0);
+      }
     }
     return acc;
   };
