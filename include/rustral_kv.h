@@ -108,9 +108,11 @@ int rkv_copy_blocks(void* k_pool, void* v_pool, int64_t layer_stride_bytes, int 
 /* Workspace (bytes) rkv_decode_attention needs for split-K partials.
  * max_context: host-side upper bound on every ctx_lens[b] (for example
  * max_blocks_per_seq*block_size).  partition_size: the size the call will
- * use (rkv_decode_partition_size_for), or <= 0 for the smallest size any
- * call picks by itself (512), which is enough for every pool dtype and
- * shape. */
+ * use (rkv_decode_partition_size_for), or <= 0 for the smallest size a call
+ * of this shape picks by itself (512; 128 or 256 for calls of one or two
+ * sequences), which is enough for every pool dtype.  A call that leaves the
+ * size to the library and brings a smaller workspace, but one that holds
+ * 512-token partitions, runs with those. */
 size_t rkv_decode_workspace_bytes(int num_seqs, int num_q_heads, int head_dim, int max_context,
                                   int partition_size);
 
@@ -125,7 +127,9 @@ int rkv_decode_partition_size(int partition_size, int head_dim, int dtype, int m
 
 /* Partition size rkv_decode_attention (and _noalloc) uses for a call of this
  * shape: the request when partition_size > 0 (rules of
- * rkv_decode_partition_size), else its own pick.  With W = num_kv_heads *
+ * rkv_decode_partition_size), else its own pick.  Above 512 tokens of
+ * max_context it is the smaller of 128 and 256 for which num_kv_heads *
+ * num_seqs * ceil(max_context / size) <= 256.  Else, with W = num_kv_heads *
  * num_seqs * max_context / 2 tokens: RKV_F32 and RKV_BF16 pools take 512
  * when W < 800 * 512, 1-byte pools when W < 1600 * 512; above that, RKV_BF16
  * pools with head_dim 128 and at most 4 query heads per KV head take 1280

@@ -254,9 +254,26 @@ int default_part(int dtype, int /*max_context*/) { return one_byte(dtype) ? kPQ 
 // 4096], 512 / 640: 8 sequences 13.4 / 15.2, 16 sequences 21.0 / 24.2, 32
 // sequences 33.0 / 33.8, 64 sequences 66.5 / 64.2; 64 x 1 KV head 16.0 /
 // 16.4).
+// Calls of one or two users: with 512-token partitions most CUs have nothing
+// to do, so the smallest of 128 and 256 tokens is taken that still gives every
+// workgroup a CU of its own (256).  us per call, partition kernel and merge,
+// 512 / 256 / 128 tokens, Llama-3-8B heads over bf16 pools: 1 sequence of 600
+// tokens 11.5 / 8.7 / 7.6, 1,000 11.5 / 8.6 / 7.9, 2,000 11.5 / 8.9 / 8.9,
+// 4,096 11.8 / 10.1 / 9.6, 16,000 16.3 / 17.9 / 19.5; U[512, 4096]: 2 sequences
+// 12.8 / 10.5 / 11.7, 4 sequences 12.7 / 14.2 / 15.5; 16 x 1 KV head 13.1 /
+// 10.5 / 12.0; int8, 1 of 4,096 11.6 / 9.1 / 9.0.  0: not such a call.  (A call
+// that fits one 512-token partition needs no merge and is left alone.)
+int tiny_part(int num_seqs, int64_t num_kv_heads, int cap) {
+  if (cap <= kSmallP) return 0;
+  for (int P = kShortP; P <= 2 * kShortP; P *= 2)
+    if (num_kv_heads * num_seqs * ((cap + P - 1) / P) <= 256) return P;
+  return 0;
+}
+
 int shape_part(int dtype, int num_seqs, int num_q_heads, int num_kv_heads, int head_dim,
                int cap) {
   if (num_kv_heads <= 0 || num_seqs <= 0 || cap <= 0) return default_part(dtype, cap);
+  if (const int tiny = tiny_part(num_seqs, num_kv_heads, cap)) return tiny;
   const double work = (double)num_kv_heads * num_seqs * (0.5 * cap);  // KV-head tokens
   if (work < (one_byte(dtype) ? 1600.0 : 800.0) * kSmallP) return kSmallP;
   if (one_byte(dtype)) return default_part(dtype, cap);
@@ -321,6 +338,18 @@ size_t ws_bytes(int B, int Hq, int D, int max_parts) {
   const size_t acc = rows * D * sizeof(float);
   const size_t acc_pad = (acc + 255) & ~size_t(255);
   return acc_pad + rows * 2 * sizeof(float);
+}
+
+// shape_part for a call with this workspace: one sized for 512-token
+// partitions (all a call once needed) still takes a call tiny_part would split
+// finer, at 512.
+int auto_part(int dtype, int num_seqs, int num_q_heads, int num_kv_heads, int head_dim, int cap,
+              size_t workspace_bytes) {
+  const int P = shape_part(dtype, num_seqs, num_q_heads, num_kv_heads, head_dim, cap);
+  if (P < kSmallP && num_q_heads > 0 && head_dim > 0 &&
+      ws_bytes(num_seqs, num_q_heads, head_dim, (cap + P - 1) / P) > workspace_bytes)
+    return kSmallP;
+  return P;
 }
 
 int ctx_cap_of(int max_context, int max_blocks_per_seq, int block_size) {
@@ -454,10 +483,11 @@ extern "C" size_t rkv_decode_workspace_bytes(int num_seqs, int num_q_heads, int 
                                              int max_context, int partition_size) {
   if (num_seqs <= 0 || num_q_heads <= 0 || head_dim <= 0 || max_context <= 0) return 0;
   // a given partition size, else the smallest size a call picks by itself
-  // (the 512-token build's, for small bf16 calls): enough for every pool
-  // dtype and shape
-  const int dflt = std::min({kSmallP, default_part(RKV_BF16, max_context),
-                             default_part(RKV_I8, max_context)});
+  // (tiny_part with as few KV heads as num_q_heads allows, else the 512-token
+  // build's): enough for every pool dtype and shape
+  const int tiny = tiny_part(num_seqs, (num_q_heads + 7) / 8, max_context);
+  const int dflt = tiny ? tiny : std::min({kSmallP, default_part(RKV_BF16, max_context),
+                                           default_part(RKV_I8, max_context)});
   const int P = partition_size > 0 ? partition_size : dflt;
   const int max_parts = (max_context + P - 1) / P;
   return ws_bytes(num_seqs, num_q_heads, head_dim, max_parts);
@@ -552,9 +582,10 @@ extern "C" int rkv_decode_attention(float* out, const float* q, const void* k_po
   const int P =
       partition_size > 0
           ? partition_size
-          : shape_part(dtype, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                       ctx_cap_of(max_context < 0 ? 0 : max_context,
-                                  max_blocks_per_seq < 0 ? 0 : max_blocks_per_seq, block_size));
+          : auto_part(dtype, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                      ctx_cap_of(max_context < 0 ? 0 : max_context,
+                                 max_blocks_per_seq < 0 ? 0 : max_blocks_per_seq, block_size),
+                      workspace ? workspace_bytes : 0);
   int rc = rkv_decode_attention_partitions(out, q, k_pool, v_pool, block_tables,
                                            max_blocks_per_seq, ctx_lens, num_seqs, num_q_heads,
                                            num_kv_heads, head_dim, block_size, num_blocks,
@@ -591,9 +622,10 @@ extern "C" int rkv_decode_attention_append(
   const int P =
       partition_size > 0
           ? partition_size
-          : shape_part(dtype, num_seqs, num_q_heads, num_kv_heads, head_dim,
-                       ctx_cap_of(max_context < 0 ? 0 : max_context,
-                                  max_blocks_per_seq < 0 ? 0 : max_blocks_per_seq, block_size));
+          : auto_part(dtype, num_seqs, num_q_heads, num_kv_heads, head_dim,
+                      ctx_cap_of(max_context < 0 ? 0 : max_context,
+                                 max_blocks_per_seq < 0 ? 0 : max_blocks_per_seq, block_size),
+                      workspace ? workspace_bytes : 0);
   DecodeArgs a{out, q, k_pool, v_pool, block_tables, max_blocks_per_seq, ctx_lens, num_seqs,
                num_q_heads, num_kv_heads, head_dim, block_size, num_blocks, max_context, scale,
                dtype, P, workspace, workspace_bytes, static_cast<hipStream_t>(stream)};

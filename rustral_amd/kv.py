@@ -209,6 +209,9 @@ def decode_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor
         # the split entry points take 640 for 0: ask for this shape's pick so
         # the two passes partition like the one-call entry point
         partition_size = partition_size_for(B, hq, hkv, d, dt, min(max_context, mbs * bs))
+        if partition_size < 512 and ws_len < workspace_bytes(B, hq, d, max_context,
+                                                             partition_size):
+            partition_size = 512  # what the one-call entry point does
     if passes in ("both", "partitions"):
         fn = lib().rkv_decode_attention if passes == "both" else lib().rkv_decode_attention_partitions
         check(fn(out.data_ptr(), q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),

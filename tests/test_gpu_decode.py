@@ -304,6 +304,33 @@ def test_decode_short_context_builds(dev, cap, dtype, hq, hkv, d):
     assert_allclose_ref(to_np(out), want, RTOL, ATOL, f"context cap {cap} vs oracle")
 
 
+@pytest.mark.parametrize("dtype", ["bf16", "f32"])
+@pytest.mark.parametrize("L0,hq,hkv,d", [(513, 32, 8, 128), (1025, 8, 4, 64), (4096, 32, 8, 128),
+                                         (5000, 16, 2, 32)])
+def test_decode_one_sequence_fine_partitions(dev, dtype, L0, hq, hkv, d):
+    """A single sequence takes 128- or 256-token partitions; a workspace that
+    only holds 512-token ones gives exactly the 512-token call, in one call
+    and as two passes."""
+    say(f"decode fine partitions L={L0} {dtype} hq={hq} hkv={hkv} d={d}")
+    ctx = np.array([L0], np.int32)
+    q, kp, vp, kf, vf, tables = case(L0 + d, 1, hq, hkv, d, ctx, dtype)
+    scale = float(np.float32(1.0 / math.sqrt(d)))
+    cap = tables.shape[1] * 16
+    code = kv._lib.RKV_BF16 if dtype == "bf16" else kv._lib.RKV_F32
+    assert kv.partition_size_for(1, hq, hkv, d, code, cap) in (128, 256)
+    args = [to_dev(x, dev) for x in (q, kp, vp, tables, ctx)]
+    want = oracle.decode_attention(q, kp, vp, tables, ctx, scale)
+    assert_allclose_ref(to_np(kv.decode_attention(*args, scale)), want, RTOL, ATOL, "own pick")
+    ws = torch.empty(kv.workspace_bytes(1, hq, d, cap, 512), dtype=torch.uint8, device=dev)
+    at512 = kv.decode_attention(*args, scale, partition_size=512)
+    assert torch.equal(kv.decode_attention(*args, scale, workspace=ws), at512)
+    out = torch.zeros_like(at512)
+    for passes in ("partitions", "merge"):
+        kv.decode_attention(*args, scale, workspace=ws, out=out, passes=passes)
+    torch.cuda.synchronize()
+    assert torch.equal(out, at512)
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (16, 2, 128), (8, 8, 64), (8, 4, 32),
                                       (64, 8, 128)])
 @pytest.mark.parametrize("P", [768, 896, 1024, 1280, 0])
