@@ -147,79 +147,118 @@ constexpr int kChunk = 64;        // features per staged chunk
 constexpr int kRow = kChunk + 4;  // LDS row stride: an odd count of 16-byte units,
                                   // so 16-byte reads of 64 rows hit distinct banks
 
-// Layer-norm statistics (mean, sqrt(var + eps)) of four rows by one wave, 16
-// lanes a row: the reference's two serial sums, whose 2 n dependent additions
-// set the time.  Terms are loaded (and squared) 64 features at a time, 16
-// lanes wide, pass through the wave's LDS buffer (2 x 4 rows of kRow floats)
-// one chunk ahead and are added in order by every lane of the row.  Measured
-// at 4,096 features: 38 us of a one-row call; handing the terms around with
-// row_newbcast instead 39 us alone but 70 us with two waves on the SIMD (the
-// moves run at a quarter of the rate), one wave adding the rows of four 44 us.
-template <bool VEC>
-__device__ __forceinline__ float2 row_stats(const float* xr, int n, float eps, float* buf) {
+// Layer-norm statistics (mean, sqrt(var + eps)) of the 4 NW rows of a
+// workgroup to s_stat: the reference's two serial sums per row, whose 2 n
+// dependent additions set the time.  Every wave loads (and squares) its four
+// rows' terms, 16 lanes a row, kStat features at a time; they pass through LDS
+// (buf: 2 x 4 NW rows of kStat + 4 floats) a piece ahead, and wave 0 adds them,
+// a lane (or a quarter wave) a row, 16 reads a burst (a wave pays some 17 cycles to turn
+// from additions to LDS reads).  64 tokens of Llama-3-8B's q / k / v: 141 us;
+// every wave adding its own four rows reads LDS four times as often, 152;
+// handing terms around with row_newbcast 171.
+constexpr int kStat = 256;
+template <bool VEC, int NW>
+__device__ __forceinline__ void row_stats(const float* xr, int n, float eps, float* buf,
+                                          float2* s_stat) {
 #pragma clang fp contract(off)
-  const int lane = threadIdx.x & 63, k4 = 4 * (lane & 15);
-  const int full = n / (4 * kChunk) * 4;  // chunks taken four at a time, unguarded
-  buf += (lane >> 4) * kRow;
+  constexpr int ROWS = 4 * NW, S = kStat + 4, U = kStat / 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, k4 = 4 * (lane & 15);
+  const int slot = 4 * wave + (lane >> 4);  // the row this lane loads for
+  float* wr = buf + slot * S + k4;
+  // the row this lane adds: with one wave the one it loads, so that its mean
+  // needs no exchange
+  const int row = NW == 1 ? slot : lane & (ROWS - 1);
+  const float* rd = buf + row * S;
+  const int whole = n / kStat;
   auto pass = [&](auto term) __attribute__((always_inline)) {
     float acc = 0.0f;
-    f32x4_t t[2][kChunk / 4];
-    auto put_chunk = [&](int i, const f32x4_t& v) __attribute__((always_inline)) {
-      float* b = buf + i * 4 * kRow;
-      *reinterpret_cast<f32x4_t*>(b + k4) = v;
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+    f32x4_t t[2][16];
+    auto read = [&](f32x4_t(&d)[16], const float* b) __attribute__((always_inline)) {
 #pragma unroll
-      for (int s = 0; s < kChunk / 4; ++s) t[i][s] = *reinterpret_cast<const f32x4_t*>(b + 4 * s);
+      for (int s = 0; s < 16; ++s) d[s] = *reinterpret_cast<const f32x4_t*>(b + 4 * s);
+      __builtin_amdgcn_sched_barrier(0);
     };
-    auto add_chunk = [&](int i) __attribute__((always_inline)) {
+    auto add = [&](const f32x4_t(&d)[16]) __attribute__((always_inline)) {
 #pragma unroll
-      for (int s = 0; s < kChunk / 4; ++s)
+      for (int s = 0; s < 16; ++s)
 #pragma unroll
-        for (int e = 0; e < 4; ++e) acc = acc + t[i][s][e];
+        for (int e = 0; e < 4; ++e) acc = acc + d[s][e];
+      __builtin_amdgcn_sched_barrier(0);
     };
-    if (full) {
-      f32x4_t v[4];
+    f32x4_t v[U];
+    if (whole) {
+      auto request = [&](int piece) __attribute__((always_inline)) {
+        const float* p = xr + (piece < whole ? piece : whole - 1) * kStat + k4;
 #pragma unroll
-      for (int u = 0; u < 4; ++u) v[u] = load4u<VEC>(xr + u * kChunk + k4);
-      auto next = [&](int u, int c) __attribute__((always_inline)) {  // chunk c from v[u]
-        put_chunk(u & 1, term(v[u]));
-        v[u] = load4u<VEC>(xr + (c + 4 < full ? c + 4 : full - 1) * kChunk + k4);
+        for (int u = 0; u < U; ++u) v[u] = load4u<VEC>(p + 64 * u);
       };
-      next(0, 0);
-      for (int c = 0; c < full; c += 4) {
+      auto stage = [&](int i) __attribute__((always_inline)) {
 #pragma unroll
-        for (int u = 0; u < 4; ++u) {  // the last round's extra chunk is not added
-          next((u + 1) & 3, c + u + 1);
-          add_chunk(u & 1);
+        for (int u = 0; u < U; ++u)
+          *reinterpret_cast<f32x4_t*>(wr + i * ROWS * S + 64 * u) = term(v[u]);
+      };
+      request(0);
+      stage(0);
+      request(1);
+      lds_barrier();
+      for (int c = 0; c < whole; ++c) {
+        stage((c + 1) & 1);  // the last round's is not added
+        request(c + 2);
+        if (wave == 0) {
+          const float* b = rd + (c & 1) * ROWS * S;
+          read(t[0], b);
+          read(t[1], b + 64);
+          add(t[0]);
+          read(t[0], b + 128);
+          add(t[1]);
+          read(t[1], b + 192);
+          add(t[0]);
+          add(t[1]);
         }
+        lds_barrier();
       }
     }
-    f32x4_t last[4];  // the chunks past full, requested together
+    const int k0 = whole * kStat;
+    if (k0 < n) {  // features past the end add +0
 #pragma unroll
-    for (int u = 0; u < 4; ++u) last[u] = load4<VEC>(xr, (full + u) * kChunk + k4, n);
+      for (int u = 0; u < U; ++u)
+        if (k0 + 64 * u < n) v[u] = load4<VEC>(xr, k0 + 64 * u + k4, n);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int k = (full + u) * kChunk;
-      if (k < n) {
-        put_chunk(0, keep4(term(last[u]), k + k4, n));
-        add_chunk(0);
+      for (int u = 0; u < U; ++u)
+        if (k0 + 64 * u < n)
+          *reinterpret_cast<f32x4_t*>(wr + 64 * u) = keep4(term(v[u]), k0 + 64 * u + k4, n);
+      lds_barrier();
+      if (wave == 0) {
+        const float* b = rd;
+        for (int k = k0; k < n; k += 128, b += 128) {
+          read(t[0], b);
+          read(t[1], b + 64);
+          add(t[0]);
+          if (k + 64 < n) add(t[1]);
+        }
       }
+      lds_barrier();
     }
     return acc;
   };
   const float mean = pass([](const f32x4_t& x) { return x; }) / (float)n;
+  float m = mean;
+  if (wave == 0) s_stat[row].x = mean;  // every lane of a row the same
+  if constexpr (NW > 1) {
+    lds_barrier();
+    m = s_stat[slot].x;
+  }
   const float vs = pass([&](const f32x4_t& x) __attribute__((always_inline)) {
     f32x4_t t;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      const float d = x[e] - mean;
+      const float d = x[e] - m;
       t[e] = d * d;
     }
     return t;
   });
-  return make_float2(mean, sqrtf(vs / (float)n + eps));
+  if (wave == 0) s_stat[row].y = sqrtf(vs / (float)n + eps);
+  lds_barrier();
 }
 
 // Lane J of each row of 16 lanes, to the whole row.
@@ -258,8 +297,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   constexpr int NL = OW * (kChunk / 4) / (64 * NW);  // float4 of weights a thread stages
   static_assert(NL * 4 * NW == OW, "staging split");
   constexpr int WB = OW * kRow;  // floats of a weight buffer
-  static_assert(3 * OW >= 8 * NW, "the statistics buffers fit the weights'");
-  __shared__ __align__(16) float s_buf[3 * WB];
+  constexpr int SB = LN ? 8 * NW * (kStat + 4) : 0;  // floats of the statistics' buffers
+  __shared__ __align__(16) float s_buf[3 * WB > SB ? 3 * WB : SB];
+  __shared__ float2 s_stat[LN ? 4 * NW : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int n = a.n, o0 = blockIdx.x * OW;
@@ -321,12 +361,9 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   for (int e = 0; e < RW; ++e) rt[e] = row_tail(a, r0 + e < a.rows ? r0 + e : a.rows - 1, oc);
   float2 st[NX];
   if constexpr (LN) {
-    const float2 s4 = row_stats<VEC>(row_of(lane >> 4), n, a.eps, s_buf + wave * 8 * kRow);
+    row_stats<VEC, NW>(row_of(lane >> 4), n, a.eps, s_buf, s_stat);
 #pragma unroll
-    for (int i = 0; i < NX; ++i) {
-      const int src = 16 * (MFMA ? lane & 3 : i);
-      st[i] = make_float2(__shfl(s4.x, src), __shfl(s4.y, src));
-    }
+    for (int i = 0; i < NX; ++i) st[i] = s_stat[4 * wave + (MFMA ? lane & 3 : i)];
     lds_barrier();  // the buffers become weights
   }
   float *cur = s_buf, *next = s_buf + WB, *spare = s_buf + 2 * WB;
@@ -463,8 +500,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // Time is set by the wave's serial chain while there is at most one wave per
 // SIMD (1,024), then grows by 18 us a wave (RW = 1) or 36 us (RW = 4): the
 // narrow split up to 1,024 of its waves, four rows a wave from 2,048 waves of
-// one row on.  With the layer norm each wave also forms its rows' sums (38 us,
-// for one row or four): four rows a wave from 1,024 (11 rows of 6,144 columns
+// one row on.  With the layer norm each workgroup also forms its rows' sums
+// (37 us, for one row or sixteen): four rows a wave from 1,024 (11 rows of 6,144 columns
 // 109 / 106, 16 rows 112 / 105; 8 rows 77 / 104).
 // Narrow calls of up to two rows take one-wave workgroups (1 row 27.3 against
 // 31.7 us), others four rows a workgroup sharing the weights (8 x 8,192 x

@@ -302,6 +302,9 @@ def test_gpu_decoder_on_a_caller_stream(dev):
     (300, 128, 4, 2, "f32", True, True),      # a prompt's rows, GQA
     (7, 256, 8, 1, "bf16", True, False),
     (5, 4096, 32, 8, "bf16", False, True),    # Llama-3-8B layer shape
+    (1, 511, 7, 1, "f32", True, True),        # the norm's sums: 256 features and a remainder
+    (6, 257, 1, 1, "bf16", True, False),      # ... one feature
+    (18, 768, 6, 2, "f32", True, True),       # ... whole pieces only
     (64, 136, 4, 4, "f32", True, True),       # 64 columns a wave, one row each
     (260, 192, 6, 2, "bf16", True, True),     # four rows a wave, an odd chunk at the end
     (700, 72, 3, 1, "f32", False, False),     # ... without the norm
