@@ -302,17 +302,19 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   __shared__ float2 s_stat[LN ? 4 * NW : 1];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int n = a.n, o0 = blockIdx.x * OW;
+  const int n = a.n;
+  const int64_t o0 = ((int64_t)blockIdx.z * gridDim.x + blockIdx.x) * OW;
+  if (o0 >= a.cols) return;  // the whole workgroup: the last row of a split grid
+  const auto col = [&](int i) __attribute__((always_inline)) {  // column o0 + i, clamped
+    return (int)(o0 + i < a.cols ? o0 + i : a.cols - 1);
+  };
   const int r0 = (blockIdx.y * NW + wave) * RW;
 
   // staging: thread t takes float4 t % 16 of columns t / 16 + 4 NW i
   const int sk = 4 * (tid & 15), so = tid >> 4;
   const float* wrow[NL];
 #pragma unroll
-  for (int i = 0; i < NL; ++i) {
-    const int o = o0 + so + 4 * NW * i;
-    wrow[i] = weight_row(a, o < a.cols ? o : a.cols - 1);
-  }
+  for (int i = 0; i < NL; ++i) wrow[i] = weight_row(a, col(so + 4 * NW * i));
   const int pairs = n / (2 * kChunk) * 2;  // chunks the pipelined loop covers
   f32x4_t wv[2][NL];
   auto wload = [&](f32x4_t(&d)[NL], int chunk) __attribute__((always_inline)) {
@@ -354,11 +356,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
   }
   // the output column and rows of this lane (duplicates and rows past the end
   // clamped: loaded, not stored)
-  const int o = o0 + lane % OW, oc = o < a.cols ? o : a.cols - 1;
-  const ColTail ct = col_tail(a, oc);
+  const int o = col(lane % OW);
+  const ColTail ct = col_tail(a, o);
   RowTail rt[RW];
 #pragma unroll
-  for (int e = 0; e < RW; ++e) rt[e] = row_tail(a, r0 + e < a.rows ? r0 + e : a.rows - 1, oc);
+  for (int e = 0; e < RW; ++e) rt[e] = row_tail(a, r0 + e < a.rows ? r0 + e : a.rows - 1, o);
   float2 st[NX];
   if constexpr (LN) {
     row_stats<VEC, NW>(row_of(lane >> 4), n, a.eps, s_buf, s_stat);
@@ -482,7 +484,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
       for (int e = 0; e < RW; ++e) acc[e] = acc[e] + p[1][t][e];  // a chunk has an even count
   }
 
-  if (lane < OW && o < a.cols) {
+  if (lane < OW && o0 + lane < a.cols) {
 #pragma unroll
     for (int e = 0; e < RW; ++e)
       if (r0 + e < a.rows) put(a, r0 + e, o, acc[e], ct, rt[e]);
@@ -510,8 +512,11 @@ template <bool VEC, bool LN>
 void launch(const ProjArgs& a, hipStream_t s) {
   auto go = [&](auto rw, auto ow, auto nw) {
     constexpr int RW = decltype(rw)::value, OW = decltype(ow)::value, NW = decltype(nw)::value;
-    const dim3 grid((unsigned)((a.cols + OW - 1) / OW),
-                    (unsigned)((a.rows + RW * NW - 1) / (RW * NW)));
+    // a grid dimension times the workgroup stays under 2^32 threads
+    const int64_t groups = ((int64_t)a.cols + OW - 1) / OW;
+    const int64_t gx = groups < (1 << 22) ? groups : (1 << 22);
+    const dim3 grid((unsigned)gx, (unsigned)((a.rows + RW * NW - 1) / (RW * NW)),
+                    (unsigned)((groups + gx - 1) / gx));
     proj_kernel<VEC, LN, RW, OW, NW><<<grid, 64 * NW, 0, s>>>(a);
   };
   constexpr std::integral_constant<int, 1> c1{};
