@@ -504,7 +504,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // narrow split up to 1,024 of its waves, four rows a wave from 2,048 waves of
 // one row on.  With the layer norm each workgroup also forms its rows' sums
 // (37 us, for one row or sixteen): four rows a wave from 1,024 (11 rows of 6,144 columns
-// 109 / 106, 16 rows 112 / 105; 8 rows 77 / 104).
+// 109 / 106, 16 rows 112 / 105; 8 rows 77 / 104; each some 3 to 10 less since
+// one wave adds a workgroup's sums).
 // Narrow calls of up to two rows take one-wave workgroups (1 row 27.3 against
 // 31.7 us), others four rows a workgroup sharing the weights (8 x 8,192 x
 // 1,024: 56.6 against 57.5).
