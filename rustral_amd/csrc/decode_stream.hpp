@@ -63,7 +63,7 @@ constexpr int kBS = 16;
 // register ring depth in 16-byte loads per lane (16-bit / fp32 pools, 1-byte
 // pools).
 #ifndef RKV_DECODE_P
-#define RKV_DECODE_P 640  // 40 blocks; 2.8% faster than 512 at configs[2], 4% for 1-byte pools
+#define RKV_DECODE_P 640  // 40 blocks; 2.8% faster than 512 at 64 x U[512, 4096], 4% for 1-byte pools
 #endif
 #ifndef RKV_DECODE_SPLIT
 #define RKV_DECODE_SPLIT 4
@@ -77,7 +77,7 @@ constexpr int kBS = 16;
 // bf16 pools at head_dim 128: bytes of unused dynamic LDS per workgroup,
 // a knob on how many workgroups share a CU (39 KiB each: four).  With the
 // streaming (nontemporal) K/V loads, four per CU beat three (14 KiB of
-// padding) by ~2% at configs[2]; with ordinary loads it was the reverse.
+// padding) by ~2% at 64 x U[512, 4096]; with ordinary loads it was the reverse.
 #ifndef RKV_DECODE_LDS_PAD_16
 #define RKV_DECODE_LDS_PAD_16 0
 #endif
@@ -105,11 +105,11 @@ constexpr int split_of() { return sizeof(T) == 1 ? RKV_DECODE_SPLIT_Q : RKV_DECO
 // 96-token slice, 6 tiles, per wave) and 1280 tokens (10 tiles per wave, the
 // 640-token build's slice); requests that are multiples of 128 above 640 run
 // on them.  Measured in one process against the 4-wave
-// 640-token build (us per call): configs[2] (64 sequences, contexts
-// U[512, 4096]) 109.0 -> 106.7 at 768 (122.8 at 1280: too few workgroups);
+// 640-token build (us per call): 64 sequences of contexts
+// U[512, 4096] 109.0 -> 106.7 at 768 (122.8 at 1280: too few workgroups);
 // 256 x U[1, 8192] 769.3 -> 736.9 at 1280; 64 x U[8192, 16384] 547.0 ->
-// 526.5; 32 x U[12288, 24576] 403.4 -> 387.1; configs[3] (8 x U[16384,
-// 65536]) 221.2 -> 214.2.  Fewer partitions per sequence mean fewer split-K
+// 526.5; 32 x U[12288, 24576] 403.4 -> 387.1; 8 x U[16384,
+// 65536] 221.2 -> 214.2.  Fewer partitions per sequence mean fewer split-K
 // partials and a cheaper merge.
 // They pay off only with enough work: at 8 x U[512, 4096] 768 was 5% slower
 // than 640, at 4 x U[16384, 32768] 1280 was 10% slower, and for 8 query
@@ -684,7 +684,7 @@ __attribute__((amdgpu_waves_per_eu(G >= 8 ? 2 : RKV_DECODE_WAVES_PER_SIMD))) voi
     uint4* tile = ring[t % R];
     // Refill the slot just consumed with tile t + R; the refill's loads issue
     // at raised wave priority, ahead of the other waves' arithmetic on the
-    // SIMD (about 1% at configs[2]).  A tile staged in LDS frees its slot
+    // SIMD (about 1% at 64 x U[512, 4096]).  A tile staged in LDS frees its slot
     // once written there, before the step's arithmetic.
     auto refill = [&]() __attribute__((always_inline)) {
       if constexpr (t + R < NT) {
