@@ -205,12 +205,11 @@ __global__ __launch_bounds__(256) void transpose_kernel(float* __restrict__ y,
     if (c0 + c < n && r0 + tx < m) y[(int64_t)(c0 + c) * m + r0 + tx] = s_t[tx][c];
 }
 
-// Four waves per row.  Without NaN: each thread scans its elements (i = t,
-// t + 256, ...) keeping the last maximum, then lanes and waves combine (larger
+// NW waves per row.  Without NaN: each thread scans its elements (i = t,
+// t + 64 NW, ...) keeping the last maximum, then lanes and waves combine (larger
 // value, or the larger index on a tie).  With a NaN anywhere the answer depends
 // on the scan order, so thread 0 repeats the reference's left-to-right scan.
-// (One wave scanned 1,000 elements in 5.8 us traced, a chain of 16 loads a
-// lane.)  EMBED: the row's winner is a token id and its embedding row (plus the
+// EMBED: the row's winner is a token id and its embedding row (plus the
 // positional one) follows in the same launch, as rkv_embed writes it.
 struct EmbedTail {
   float* x;            // [dim]
@@ -219,20 +218,20 @@ struct EmbedTail {
   int dim;
 };
 
-template <bool EMBED>
-__global__ __launch_bounds__(256) void argmax_kernel(int32_t* __restrict__ out,
-                                                     const float* __restrict__ x, int n,
-                                                     EmbedTail tail) {
+template <int NW, bool EMBED>
+__global__ __launch_bounds__(64 * NW) void argmax_kernel(int32_t* __restrict__ out,
+                                                         const float* __restrict__ x, int n,
+                                                         EmbedTail tail) {
 #pragma clang fp contract(off)
-  __shared__ float s_v[4];
-  __shared__ int s_i[4], s_nan[4], s_best;
+  __shared__ float s_v[NW];
+  __shared__ int s_i[NW], s_nan[NW], s_best;
   const int r = blockIdx.x, t = threadIdx.x, lane = t & 63, w = t >> 6;
   const float* xr = x + (int64_t)r * n;
   bool nan = false;
   float bv = -INFINITY;
   int bi = -1;
 #pragma unroll 4
-  for (int i = t; i < n; i += 256) {
+  for (int i = t; i < n; i += 64 * NW) {
     const float v = xr[i];
     nan |= v != v;
     if (bi < 0 || v >= bv) {
@@ -251,31 +250,35 @@ __global__ __launch_bounds__(256) void argmax_kernel(int32_t* __restrict__ out,
     const float ov = __shfl_xor(bv, o);
     merge(ov, __shfl_xor(bi, o));
   }
-  const bool any = __ballot(nan) != 0;
-  if (lane == 0) {
-    s_v[w] = bv;
-    s_i[w] = bi;
-    s_nan[w] = any;
+  bool any = __ballot(nan) != 0;
+  if constexpr (NW > 1) {
+    if (lane == 0) {
+      s_v[w] = bv;
+      s_i[w] = bi;
+      s_nan[w] = any;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NW; ++k) any |= s_nan[k] != 0;
   }
-  __syncthreads();
   if (t == 0) {
     int best;
-    if (s_nan[0] | s_nan[1] | s_nan[2] | s_nan[3]) {
+    if (any) {
       best = 0;
       for (int i = 1; i < n; ++i)
         if (!(xr[best] > xr[i])) best = i;
     } else {
 #pragma unroll
-      for (int k = 1; k < 4; ++k) merge(s_v[k], s_i[k]);
+      for (int k = 1; k < NW; ++k) merge(s_v[k], s_i[k]);
       best = bi;
     }
     out[r] = best;
-    s_best = best;
+    if constexpr (EMBED) s_best = best;
   }
   if constexpr (EMBED) {
     __syncthreads();
     const float* row = tail.table + (int64_t)s_best * tail.dim;
-    for (int i = t; i < tail.dim; i += 256) tail.x[i] = row[i] + tail.pe[i];
+    for (int i = t; i < tail.dim; i += 64 * NW) tail.x[i] = row[i] + tail.pe[i];
   }
 }
 
@@ -285,7 +288,7 @@ unsigned blocks_for(int64_t n, int per) { return (unsigned)((n + per - 1) / per)
 
 int argmax_embed_launch(int32_t* id, float* x_next, const float* logits, int vocab,
                         const float* table, const float* pe_row, int dim, hipStream_t s) {
-  argmax_kernel<true><<<1, 256, 0, s>>>(id, logits, vocab, EmbedTail{x_next, table, pe_row, dim});
+  argmax_kernel<4, true><<<1, 256, 0, s>>>(id, logits, vocab, EmbedTail{x_next, table, pe_row, dim});
   return check_launch("argmax_embed");
 }
 
@@ -402,7 +405,14 @@ extern "C" int rkv_argmax(int32_t* out, const float* x, int rows, int n, void* s
   if (rows < 0 || n <= 0) return fail(RKV_ERR_INVALID_ARG, "rkv_argmax: bad size argument");
   if (rows == 0) return RKV_OK;
   if (!out || !x) return fail(RKV_ERR_INVALID_ARG, "rkv_argmax: null pointer argument");
-  argmax_kernel<false><<<(unsigned)rows, 256, 0, static_cast<hipStream_t>(stream)>>>(out, x, n,
-                                                                                     EmbedTail{});
+  const hipStream_t s = static_cast<hipStream_t>(stream);
+  // Four waves cut a long row's chain of loads (us, four / one: 1 row of 4,096
+  // 3.9 / 5.5, of 32,000 9.4 / 25.6); up to 1,024 columns they only cost
+  // workgroups (1 x 1,000 3.6 / 3.7; 4,096 x 256 6.7 / 4.3; 65,536 x 100 51 /
+  // 19).  2^24 rows of four waves would be 2^32 threads, at which a grid wraps.
+  if (n <= 1024 || rows >= 1 << 24)
+    argmax_kernel<1, false><<<(unsigned)rows, 64, 0, s>>>(out, x, n, EmbedTail{});
+  else
+    argmax_kernel<4, false><<<(unsigned)rows, 256, 0, s>>>(out, x, n, EmbedTail{});
   return check_launch("rkv_argmax");
 }

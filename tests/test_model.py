@@ -385,6 +385,35 @@ def test_gpu_argmax_matches_reference_rule(torch_dev):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 1024, 1025, 2500])
+def test_gpu_argmax_row_lengths(torch_dev, n):
+    """Rows on both sides of the one-wave / four-wave line and at the waves'
+    edges: random, tied, all -inf and NaN at either end."""
+    torch, dev = torch_dev
+    rng = np.random.default_rng(n)
+    rows = [rng.standard_normal(n), rng.integers(-2, 3, n), np.full(n, -np.inf)]
+    for at in (0, n // 2, n - 1):
+        r = rng.standard_normal(n)
+        r[at] = np.nan
+        rows.append(r)
+    x = np.stack(rows).astype(np.float32)
+    got = model.argmax(torch.from_numpy(x).to(dev)).cpu().numpy()
+    assert got.tolist() == [oracle.argmax(r) for r in x]
+
+
+@pytest.mark.gpu
+def test_gpu_argmax_more_rows_than_a_four_wave_grid(torch_dev):
+    """2^24 rows and more: with four waves a row the grid would be 2^32 threads,
+    at which it wraps and rows stay unwritten."""
+    torch, dev = torch_dev
+    rows = 2**24 + 3
+    x = torch.zeros((rows, 2), device=dev)
+    want = torch.arange(rows, dtype=torch.int32, device=dev) % 2
+    x[want == 0, 0] = 1.0
+    assert torch.equal(model.argmax(x), want)
+
+
+@pytest.mark.gpu
 def test_gpu_softmax_dim_matches_oracle(torch_dev):
     """rkv_softmax_dim against the oracle's softmax_dim: the reference's golden
     rows at its tolerance (crates/core/tests/golden_microblock_ops.rs:14-26,
