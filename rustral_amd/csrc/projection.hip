@@ -508,7 +508,11 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2))) vo
 // one wave adds a workgroup's sums).
 // Narrow calls of up to two rows take one-wave workgroups (1 row 27.3 against
 // 31.7 us), others four rows a workgroup sharing the weights (8 x 8,192 x
-// 1,024: 56.6 against 57.5).
+// 1,024: 56.6 against 57.5).  One row takes them at any width, since three of
+// four waves of a wider split have no row: 128,256 columns, 1 x 16 columns / 1 x
+// 64 / 4 x 64 [before]: n = 4,096 380 / 428 / 451 [427], 512 42.7 / 43.1 / 51.1
+// [45.4], 128 13.5 / 14.7 / 17.9 [13.3]; with the layer norm, 128,000 columns, n =
+// 4,096 463 / 497 / 576 [618].
 template <bool VEC, bool LN>
 void launch(const ProjArgs& a, hipStream_t s) {
   auto go = [&](auto rw, auto ow, auto nw) {
@@ -526,7 +530,7 @@ void launch(const ProjArgs& a, hipStream_t s) {
   constexpr std::integral_constant<int, 64> c64{};
   const int64_t rows = a.rows, rows4 = (rows + 3) / 4 * 4;
   const int64_t narrow = ((int64_t)a.cols + 15) / 16, wide = ((int64_t)a.cols + 63) / 64;
-  if (narrow * rows <= 1024)
+  if (rows == 1 || narrow * rows <= 1024)
     rows <= 2 ? go(c1, c16, c1) : go(c1, c16, c4);
   else if (wide * rows4 <= (LN ? 1024 : 2048))
     go(c1, c64, c4);

@@ -223,6 +223,7 @@ def test_gpu_linear_bit_exact(torch_dev, rows, i, o):
 @pytest.mark.gpu
 @pytest.mark.parametrize("rows,i,o,skew", [
     (1, 1, 1, 0), (2, 129, 17, 0),            # 16 columns a wave, one-wave workgroups
+    (1, 192, 16400, 0), (1, 131, 40003, 1),   # ... one row at any width
     (3, 64, 16, 0), (7, 191, 200, 1),         # ... four rows a workgroup; rows not 16-byte aligned
     (16, 1024, 1025, 0), (6, 128, 2800, 0),   # 64 columns a wave, one row each
     (9, 63, 4111, 3), (64, 256, 2048, 0),
