@@ -254,19 +254,29 @@ int default_part(int dtype, int /*max_context*/) { return one_byte(dtype) ? kPQ 
 // 4096], 512 / 640: 8 sequences 13.4 / 15.2, 16 sequences 21.0 / 24.2, 32
 // sequences 33.0 / 33.8, 64 sequences 66.5 / 64.2; 64 x 1 KV head 16.0 /
 // 16.4).
-// Calls of one or two users: with 512-token partitions most CUs have nothing
-// to do, so the smallest of 128 and 256 tokens is taken that still gives every
-// workgroup a CU of its own (256).  us per call, partition kernel and merge,
-// 512 / 256 / 128 tokens, Llama-3-8B heads over bf16 pools: 1 sequence of 600
-// tokens 11.5 / 8.7 / 7.6, 1,000 11.5 / 8.6 / 7.9, 2,000 11.5 / 8.9 / 8.9,
-// 4,096 11.8 / 10.1 / 9.6, 16,000 16.3 / 17.9 / 19.5; U[512, 4096]: 2 sequences
-// 12.8 / 10.5 / 11.7, 4 sequences 12.7 / 14.2 / 15.5; 16 x 1 KV head 13.1 /
-// 10.5 / 12.0; int8, 1 of 4,096 11.6 / 9.1 / 9.0.  0: not such a call.  (A call
-// that fits one 512-token partition needs no merge and is left alone.)
+// Calls with few workgroups: 512-token partitions leave most CUs idle, so the
+// smaller of 128 and 256 tokens is taken that gives at most 256 workgroups (a CU
+// each) and at most 128 partitions a sequence.  us per call, partition kernel and
+// merge, at 512 tokens / the pick; bf16 pools, head_dim 128, contexts at the cap
+// unless given:
+//   8 KV heads x 4: 1 sequence of 600 11.5 / 7.6, 4,096 11.8 / 9.6; 2 of U[512,
+//   4096] 12.8 / 10.5; 4 of 600 12.3 / 8.7, 1,024 12.0 / 9.2, 2,048 12.6 / 11.6; 8
+//   of 600 12.4 / 10.0, 1,024 12.6 / 11.3; 10 of 700 13.0 / 11.3.
+//   1 x 4: 1 of 16,384 12.6 / 10.3, 32,768 13.3 / 11.6; 16 of 2,048 12.5 / 10.7,
+//   4,096 13.4 / 13.0; 64 of 600 12.9 / 10.8, 1,024 13.0 / 12.3; 85 of 700 13.3 /
+//   12.1.  2 x 4: 1 of 32,768 13.9 / 13.7; 32 of 1,024 12.9 / 12.1.  32 x 1: 1 of
+//   1,024 10.7 / 8.7, 2 of 1,024 11.5 / 10.6.
+// Outside it: 4 of U[512, 4096] 12.7 / 14.2 at 256, 1 of 16,000 16.3 / 17.9; one KV
+// head at 65,536 tokens 14.6 / 15.3 at 256 (256 partials to a merge workgroup).
+// 0: not such a call.  (One that fits a 512-token partition needs no merge and is
+// left alone.)
+constexpr int kTinyGroups = 256, kTinyParts = 128;
 int tiny_part(int num_seqs, int64_t num_kv_heads, int cap) {
   if (cap <= kSmallP) return 0;
-  for (int P = kShortP; P <= 2 * kShortP; P *= 2)
-    if (num_kv_heads * num_seqs * ((cap + P - 1) / P) <= 256) return P;
+  for (int P = kShortP; P <= 2 * kShortP; P *= 2) {
+    const int64_t parts = ((int64_t)cap + P - 1) / P;
+    if (parts <= kTinyParts && num_kv_heads * num_seqs * parts <= kTinyGroups) return P;
+  }
   return 0;
 }
 

@@ -128,8 +128,8 @@ def test_workspace_size():
     assert F(0, 1, 32, 8, 128, RKV_BF16, 191999) == 640
     assert F(0, 1, 32, 8, 128, RKV_BF16, 102400) == 640   # 8 * 51200 = 800 x 512
     assert F(0, 1, 32, 8, 128, RKV_BF16, 102399) == 512
-    # one or two sequences: the smaller of 128 and 256 that leaves at most 256
-    # workgroups; one partition of up to 512 tokens stays one
+    # few workgroups: the smaller of 128 and 256 that leaves at most 256 of them;
+    # one partition of up to 512 tokens stays one
     for dt in (RKV_F32, RKV_BF16, RKV_I8, RKV_FP8):
         assert F(0, 1, 32, 8, 128, dt, 512) == 512
         assert F(0, 1, 32, 8, 128, dt, 513) == 128
@@ -140,6 +140,12 @@ def test_workspace_size():
         assert F(0, 1, 32, 8, 128, dt, 8192) == 256
         assert F(0, 1, 32, 8, 128, dt, 8193) == 512
         assert F(0, 16, 4, 1, 128, dt, 4096) == 256
+        # ... and at most 128 partitions a sequence (one KV head)
+        assert F(0, 1, 4, 1, 128, dt, 16384) == 128
+        assert F(0, 1, 4, 1, 128, dt, 16385) == 256
+        assert F(0, 1, 4, 1, 128, dt, 32768) == 256
+        assert F(0, 1, 4, 1, 128, dt, 32769) == 512
+        assert F(0, 2, 4, 1, 128, dt, 32768) == 256
     # ... and the default workspace covers them for any group size
     for B, hq, hkv, maxc in ((1, 32, 8, 4096), (1, 32, 4, 8192), (2, 32, 32, 600), (3, 8, 1, 5000),
                              (1, 1, 1, 32768)):
