@@ -108,9 +108,9 @@ int rkv_copy_blocks(void* k_pool, void* v_pool, int64_t layer_stride_bytes, int 
 /* Workspace (bytes) rkv_decode_attention needs for split-K partials.
  * max_context: host-side upper bound on every ctx_lens[b] (for example
  * max_blocks_per_seq*block_size).  partition_size: the size the call will
- * use (rkv_decode_partition_size_for), or <= 0 for the smallest size a call
- * of this shape picks by itself (512; 128 or 256 for calls of one or two
- * sequences), which is enough for every pool dtype.  A call that leaves the
+ * use (rkv_decode_partition_size_for), or <= 0 for what any call of this many
+ * sequences and heads picks by itself at up to max_context tokens, whatever
+ * its pool dtype, number of KV heads and context cap.  A call that leaves the
  * size to the library and brings a smaller workspace, but one that holds
  * 512-token partitions, runs with those. */
 size_t rkv_decode_workspace_bytes(int num_seqs, int num_q_heads, int head_dim, int max_context,

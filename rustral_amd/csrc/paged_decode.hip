@@ -492,14 +492,19 @@ using namespace rkv;
 extern "C" size_t rkv_decode_workspace_bytes(int num_seqs, int num_q_heads, int head_dim,
                                              int max_context, int partition_size) {
   if (num_seqs <= 0 || num_q_heads <= 0 || head_dim <= 0 || max_context <= 0) return 0;
-  // a given partition size, else the smallest size a call picks by itself
-  // (tiny_part with as few KV heads as num_q_heads allows, else the 512-token
-  // build's): enough for every pool dtype and shape
-  const int tiny = tiny_part(num_seqs, (num_q_heads + 7) / 8, max_context);
-  const int dflt = tiny ? tiny : std::min({kSmallP, default_part(RKV_BF16, max_context),
-                                           default_part(RKV_I8, max_context)});
-  const int P = partition_size > 0 ? partition_size : dflt;
-  const int max_parts = (max_context + P - 1) / P;
+  // a given partition size, else the most partitions any pick gives a call of up
+  // to max_context tokens: the 512-token build's, or tiny_part's at as few KV
+  // heads as num_q_heads allows
+  const auto parts = [&](int64_t P) { return (max_context + P - 1) / P; };
+  if (partition_size > 0)
+    return ws_bytes(num_seqs, num_q_heads, head_dim, (int)parts(partition_size));
+  const int64_t groups = (int64_t)num_seqs * ((num_q_heads + (int64_t)7) / 8);
+  const int64_t tiny =
+      max_context <= kSmallP
+          ? 1
+          : std::min({parts(kShortP), (int64_t)kTinyParts, (int64_t)kTinyGroups / groups});
+  static_assert(kSmallP <= kP && kSmallP <= kPQ, "512 tokens is the smallest pick but tiny_part's");
+  const int max_parts = (int)std::max(parts(kSmallP), tiny);
   return ws_bytes(num_seqs, num_q_heads, head_dim, max_parts);
 }
 

@@ -152,6 +152,15 @@ def test_workspace_size():
         P = F(0, B, hq, hkv, 128, RKV_BF16, maxc)
         assert (L.rkv_decode_workspace_bytes(B, hq, 128, maxc, 0)
                 >= L.rkv_decode_workspace_bytes(B, hq, 128, maxc, P))
+    # ... also where the call's context cap (its block table) is below the
+    # max_context the workspace is sized with
+    for B, hq, hkv, maxc in ((1, 64, 8, 4097), (1, 32, 8, 8193), (2, 64, 8, 4200), (16, 8, 1, 4097),
+                             (1, 8, 1, 65536), (3, 32, 32, 1100), (4, 16, 4, 1 << 20)):
+        ws = L.rkv_decode_workspace_bytes(B, hq, 128, maxc, 0)
+        for cap in sorted({c for c in range(16, maxc, 16) if c < 9000} | {16384, 32768, 65536, maxc}):
+            if cap <= maxc:
+                P = F(0, B, hq, hkv, 128, RKV_BF16, cap)
+                assert ws >= L.rkv_decode_workspace_bytes(B, hq, 128, cap, P), (B, hq, hkv, maxc, cap)
     # the default workspace covers the smallest pick
     for maxc in (4096, 65536):
         assert (L.rkv_decode_workspace_bytes(8, 32, 128, maxc, 0)
