@@ -207,11 +207,13 @@ def decode_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor
     s = _stream(q)
     if passes != "both" and partition_size <= 0:
         # the split entry points take 640 for 0: ask for this shape's pick so
-        # the two passes partition like the one-call entry point
-        partition_size = partition_size_for(B, hq, hkv, d, dt, min(max_context, mbs * bs))
-        if partition_size < 512 and ws_len < workspace_bytes(B, hq, d, max_context,
-                                                             partition_size):
-            partition_size = 512  # what the one-call entry point does
+        # the two passes partition like the one-call entry point, which goes by
+        # the smaller of max_context and the table's tokens and takes 512 where
+        # the workspace does not hold a finer pick
+        cap = min(max_context, mbs * bs)
+        partition_size = partition_size_for(B, hq, hkv, d, dt, cap)
+        if partition_size < 512 and ws_len < workspace_bytes(B, hq, d, cap, partition_size):
+            partition_size = 512
     if passes in ("both", "partitions"):
         fn = lib().rkv_decode_attention if passes == "both" else lib().rkv_decode_attention_partitions
         check(fn(out.data_ptr(), q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(),

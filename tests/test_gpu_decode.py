@@ -331,6 +331,31 @@ def test_decode_one_sequence_fine_partitions(dev, dtype, L0, hq, hkv, d):
     assert torch.equal(out, at512)
 
 
+@pytest.mark.parametrize("maxc,ws_for", [(8192, (4096, 128)), (8192, (4096, 512)), (4097, None),
+                                         (100000, None), (8192, (4096, 256))])
+def test_decode_two_passes_partition_like_one_call(dev, maxc, ws_for):
+    """max_context above the block table's 4,096 tokens: the two passes judge a
+    caller's workspace by the smaller of the two, as the one call does, and give
+    its bits; the default workspace holds the call's own pick."""
+    hq, hkv, d, cap = 32, 8, 128, 4096
+    say(f"decode two passes max_context={maxc} workspace for {ws_for}")
+    q, kp, vp, kf, vf, tables = case(maxc, 1, hq, hkv, d, np.array([cap], np.int32), "bf16")
+    args = [to_dev(x, dev) for x in (q, kp, vp, tables, np.array([cap], np.int32))]
+    scale = float(np.float32(1.0 / math.sqrt(d)))
+    need = (kv.workspace_bytes(1, hq, d, *ws_for) if ws_for
+            else kv.workspace_bytes(1, hq, d, maxc))
+    ws = torch.empty(need, dtype=torch.uint8, device=dev)
+    common = dict(max_context=maxc, workspace=ws)
+    want = kv.decode_attention(*args, scale, **common)
+    P = 512 if ws_for and ws_for[1] > 128 else 128
+    assert torch.equal(want, kv.decode_attention(*args, scale, max_context=maxc, partition_size=P))
+    out = torch.zeros_like(want)
+    for passes in ("partitions", "merge"):
+        kv.decode_attention(*args, scale, out=out, passes=passes, **common)
+    torch.cuda.synchronize()
+    assert torch.equal(out, want)
+
+
 @pytest.mark.parametrize("hq,hkv,d", [(32, 8, 128), (16, 2, 128), (8, 8, 64), (8, 4, 32),
                                       (64, 8, 128)])
 @pytest.mark.parametrize("P", [768, 896, 1024, 1280, 0])
