@@ -136,7 +136,8 @@ int rkv_decode_partition_size(int partition_size, int head_dim, int dtype, int m
  * query heads per KV head take 1280 when W >= 1200 * 1280, else 768 when W >=
  * 1000 * 768, else 640; every other shape and dtype 640.  The split entry
  * points take this value as their partition_size to match the one-call entry
- * point. */
+ * point.  For 1-byte pools the value is one to ask rkv_decode_attention_q for:
+ * left to itself it takes 640. */
 int rkv_decode_partition_size_for(int partition_size, int num_seqs, int num_q_heads,
                                   int num_kv_heads, int head_dim, int dtype, int max_context);
 
@@ -265,8 +266,9 @@ int rkv_gather_q(float* k_out, float* v_out, const void* k_pool, const void* v_p
 
 /* rkv_decode_attention over 1-byte pools: the same result as decode on the
  * dequantized values (scores = (q . bytes) * scale * row scale; the V row
- * scale multiplies the softmax weight).  head_dim 64 or 128; workspace as
- * rkv_decode_workspace_bytes. */
+ * scale multiplies the softmax weight).  head_dim 64 or 128; partition_size <=
+ * 0 is 640 (a small call may ask for rkv_decode_partition_size_for's size);
+ * workspace as rkv_decode_workspace_bytes for that size. */
 int rkv_decode_attention_q(float* out, const float* q, const void* k_pool, const void* v_pool,
                            const float* k_scale, const float* v_scale,
                            const int32_t* block_tables, int max_blocks_per_seq,

@@ -250,10 +250,14 @@ int default_part(int dtype, int /*max_context*/) { return one_byte(dtype) ? kPQ 
 // us at 8 and 16 sequences x 8 KV heads, G = 8: 21.9 / 23.7, 32.0 / 37.1;
 // head_dim 64: 13.5 / 15.1, 20.6 / 23.6; fp32 pools: 31.8 / 37.3, 58.9 /
 // 69.0; at 32 and 64 sequences even or 640 ahead (G = 8 at 64: 121.6 /
-// 116.3).  1-byte pools take it up to twice the work (int8, contexts U[512,
+// 116.3).
+// For 1-byte pools the answer is a size for the caller to ask for (their entry
+// points take 640 otherwise): 512 up to twice the work (int8, contexts U[512,
 // 4096], 512 / 640: 8 sequences 13.4 / 15.2, 16 sequences 21.0 / 24.2, 32
 // sequences 33.0 / 33.8, 64 sequences 66.5 / 64.2; 64 x 1 KV head 16.0 /
-// 16.4).
+// 16.4).  It is no default because it does not hold for every shape: over 404
+// shapes of int8 and fp8 it took 0.64 to 1.24 of the time at 640 (median 0.83;
+// 128 x U[512, 4096] with one KV head of 64 x 8 queries 21.2 -> 25.4).
 // Calls with few workgroups: 512-token partitions leave most CUs idle, so the
 // smaller of 128 and 256 tokens is taken that gives at most 256 workgroups (a CU
 // each) and at most 128 partitions a sequence.  us per call, partition kernel and

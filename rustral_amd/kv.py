@@ -166,7 +166,8 @@ def partition_size(dtype_code: int, max_context: int, requested: int = 0, head_d
 def partition_size_for(num_seqs: int, num_q_heads: int, num_kv_heads: int, head_dim: int,
                        dtype_code: int, max_context: int, requested: int = 0) -> int:
     """The partition size decode_attention uses for a call of this shape (a
-    request <= 0: the library's pick)."""
+    request <= 0: the library's pick).  With a 1-byte dtype: a size to ask
+    decode_attention_q for."""
     p = lib().rkv_decode_partition_size_for(requested, num_seqs, num_q_heads, num_kv_heads,
                                             head_dim, dtype_code, max_context)
     check(min(p, 0))
@@ -183,7 +184,7 @@ def decode_attention(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tensor
     passes: "both" (default), "partitions" or "merge" (the two launches of
     the split-K algorithm, for callers that time or schedule them apart).
     partition_size: tokens per split-K partition (a multiple of 64 up to
-    640; 0: the library's default for max_context).
+    640, over bf16 pools of 128 up to 1280; 0: partition_size_for's pick).
     """
     _dev(q, "q", torch.float32), _dev(k_pool, "k_pool"), _dev(v_pool, "v_pool")
     _dev(block_tables, "block_tables", torch.int32), _dev(ctx_lens, "ctx_lens", torch.int32)
@@ -280,6 +281,15 @@ def _qcode(fmt) -> int:
     return _QFMT[fmt]
 
 
+def _workspace_bytes_q(num_seqs: int, num_q_heads: int, head_dim: int, max_context: int,
+                       size: int, fmt) -> int:
+    """The workspace of a call over 1-byte pools, which take the split entry
+    points' size, not partition_size_for's, where none is asked for."""
+    if size <= 0:
+        size = partition_size(_qcode(fmt), max_context, head_dim=head_dim)
+    return workspace_bytes(num_seqs, num_q_heads, head_dim, max_context, size)
+
+
 def append_q(k_pool: torch.Tensor, v_pool: torch.Tensor, k_scale: torch.Tensor,
              v_scale: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor,
              slot_mapping: torch.Tensor, fmt: str = "int8") -> None:
@@ -353,7 +363,8 @@ def decode_attention_append_q(q: torch.Tensor, k_pool: torch.Tensor, v_pool: tor
                               workspace: torch.Tensor | None = None,
                               partition_size: int = 0) -> torch.Tensor:
     """decode_attention_append over 1-byte pools: the new rows quantized as
-    append_q quantizes them, then decode_attention_q, in one launch."""
+    append_q quantizes them, then decode_attention_q, in one launch.
+    partition_size 0: 640 (see decode_attention_q)."""
     _dev(q, "q", torch.float32), _dev(k_pool, "k_pool", torch.uint8)
     _dev(v_pool, "v_pool", torch.uint8), _dev(k_scale, "k_scale", torch.float32)
     _dev(v_scale, "v_scale", torch.float32)
@@ -372,7 +383,7 @@ def decode_attention_append_q(q: torch.Tensor, k_pool: torch.Tensor, v_pool: tor
     if out is None:
         out = torch.empty_like(q)
     if workspace is None:  # a caller's is checked by the library
-        need = workspace_bytes(B, hq, d, max_context, partition_size)
+        need = _workspace_bytes_q(B, hq, d, max_context, partition_size, fmt)
         if need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     ws_ptr = workspace.data_ptr() if workspace is not None else None
@@ -390,7 +401,9 @@ def decode_attention_q(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tens
                        ctx_lens: torch.Tensor, scale: float | None = None, fmt: str = "int8", *,
                        max_context: int | None = None, out: torch.Tensor | None = None,
                        workspace: torch.Tensor | None = None, partition_size: int = 0) -> torch.Tensor:
-    """decode_attention over 1-byte pools with per-row scales."""
+    """decode_attention over 1-byte pools with per-row scales.
+    partition_size 0: 640; partition_size_for gives the size to ask for where a
+    small call wants finer partitions."""
     _dev(q, "q", torch.float32), _dev(k_pool, "k_pool", torch.uint8)
     _dev(v_pool, "v_pool", torch.uint8), _dev(k_scale, "k_scale", torch.float32)
     _dev(v_scale, "v_scale", torch.float32)
@@ -406,7 +419,7 @@ def decode_attention_q(q: torch.Tensor, k_pool: torch.Tensor, v_pool: torch.Tens
     if out is None:
         out = torch.empty_like(q)
     if workspace is None:  # a caller's is checked by the library
-        need = workspace_bytes(B, hq, d, max_context, partition_size)
+        need = _workspace_bytes_q(B, hq, d, max_context, partition_size, fmt)
         if need:
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
     ws_ptr = workspace.data_ptr() if workspace is not None else None

@@ -346,6 +346,38 @@ def test_decode_q_caller_partition_sizes(dev, fmt, P):
     assert_allclose_ref(to_np(out), want, RTOL, ATOL, f"1-byte partition {P} vs oracle")
 
 
+@pytest.mark.parametrize("fmt", ["int8", "fp8"])
+@pytest.mark.parametrize("L0", [700, 4096])
+def test_decode_q_default_partition_size(dev, monkeypatch, fmt, L0):
+    """The 1-byte entry points take 640-token partitions unless asked: the bits
+    of partition_size 640, plain and with the append, and no workspace beyond
+    what those need (rkv_decode_partition_size_for names a finer size for the
+    caller to ask for)."""
+    say(f"decode_q default partition size L={L0} fmt={fmt}")
+    rng = np.random.default_rng(L0)
+    hq, hkv, bs, d = 32, 8, 16, 128
+    ctx = np.array([L0], np.int32)
+    nb = -(-L0 // bs) + 2
+    kp, vp, ks, vs = (to_dev(x, dev) for x in quant_case(L0, nb, hkv, bs, d, fmt))
+    tables = make_tables(rng, ctx, bs, nb)
+    cap = tables.shape[1] * bs
+    q, kn, vn = (to_dev(rng.standard_normal((1, h, d)).astype(np.float32), dev)
+                 for h in (hq, hkv, hkv))
+    td, cd = to_dev(tables, dev), to_dev(ctx, dev)
+    assert kv.partition_size_for(1, hq, hkv, d, CODE[fmt], cap) == 128
+    sizes = []
+    real = kv.workspace_bytes
+    monkeypatch.setattr(kv, "workspace_bytes", lambda *a: sizes.append(real(*a)) or sizes[-1])
+    outs = []
+    for P in (0, 640):
+        outs.append(kv.decode_attention_append_q(q, kp, vp, ks, vs, kn, vn, td, cd, None, fmt,
+                                                 partition_size=P))
+        outs.append(kv.decode_attention_q(q, kp, vp, ks, vs, td, cd, None, fmt, partition_size=P))
+    torch.cuda.synchronize()
+    assert all(torch.equal(o, outs[0]) for o in outs)
+    assert set(sizes) == {real(1, hq, d, cap, 640)}
+
+
 @pytest.mark.parametrize("P", [0, 256, 640])
 @pytest.mark.parametrize("max_context", [None, 1000])
 @pytest.mark.parametrize("fmt", ["int8", "fp8"])
