@@ -23,10 +23,15 @@ def _dtype_code(t: torch.Tensor) -> int:
     raise TypeError(f"KV pool dtype {t.dtype}: want float32 or bfloat16")
 
 
+# The raw handle of a device's current stream without building the Stream object
+# (1.7 of a small call's 8 us on the host); a private name, so a torch without it
+# takes the public way.
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (
+    lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+
 def _stream(t: torch.Tensor) -> int:
-    # the raw handle of torch.cuda.current_stream(t.device), without building
-    # the Stream object (1.7 of a small call's 8 us on the host)
-    return torch._C._cuda_getCurrentRawStream(t.get_device())
+    return _raw_stream(t.get_device())
 
 
 def _dev(t: torch.Tensor, name: str, dtype=None) -> torch.Tensor:

@@ -309,3 +309,32 @@ def test_decode_append_q_rejects_bad_arguments():
     assert call(vn=8) == RKV_ERR_INVALID_ARG
     assert call(d=32) == RKV_ERR_UNSUPPORTED
     assert call(dt=RKV_FP8, d=48) == RKV_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("private", [True, False])
+def test_front_end_stream_handle(monkeypatch, private):
+    """The front end's stream handle is the device's current one with torch's
+    private raw-handle function and without it."""
+    import importlib.util
+    import torch
+    from rustral_amd import kv
+
+    class Stream:
+        cuda_stream = 77
+
+    name = "_cuda_getCurrentRawStream"
+    if private:
+        monkeypatch.setattr(torch._C, name, lambda device: 70 + device, raising=False)
+    else:
+        monkeypatch.delattr(torch._C, name, raising=False)
+    monkeypatch.setattr(torch.cuda, "current_stream",
+                        lambda device: Stream() if device == 7 else None)
+    spec = importlib.util.spec_from_file_location("rustral_amd.kv_reloaded", kv.__file__)
+    mod = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(mod)
+
+    class Tensor:
+        def get_device(self):
+            return 7
+
+    assert mod._stream(Tensor()) == 77
