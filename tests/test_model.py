@@ -232,8 +232,8 @@ def test_gpu_linear_bit_exact(torch_dev, rows, i, o):
 def test_gpu_linear_splits_bit_exact(torch_dev, rows, i, o, skew):
     """Every split of the projection kernel at the edges of its chunks (64
     features, pairs of them unguarded), column groups and row groups: equal to
-    the oracle's serial sums bit for bit, with exact zeros, denormal products
-    and sums that cancel among the terms."""
+    the oracle's serial sums bit for bit, with exact zeros of both signs and
+    terms of very different size (sums of denormals: the test below)."""
     torch, dev = torch_dev
     rng = np.random.default_rng(rows * 1000 + i + o)
     x = rng.standard_normal((rows, i)).astype(np.float32)
@@ -251,6 +251,66 @@ def test_gpu_linear_splits_bit_exact(torch_dev, rows, i, o, skew):
 
     got = model.linear(t(x), t(w)).cpu().numpy()
     assert np.array_equal(got, oracle.linear(x, w))
+
+
+def denormal_linear_case(rows, i, o):
+    """x [rows, i], w [o, i] whose sums hold denormal terms only, once a pair
+    +a, -a has cancelled in rows 0, 3, ...: products of normal numbers down to
+    below the smallest denormal (rows 0, 1, 3, 4, ...), and of denormal weights
+    (rows 2, 5, ... and every fourth column)."""
+    rng = np.random.default_rng(7 * rows + i + o)
+    x = rng.standard_normal((rows, i)).astype(np.float32)
+    w = (rng.standard_normal((o, i)) * np.exp2(rng.uniform(-81, -58, (o, i)))).astype(np.float32)
+    w[3::4] = (rng.standard_normal((len(w[3::4]), i)) * 2.0**-134).astype(np.float32)
+    x[0::3] *= np.float32(2.0**-70)
+    x[1::3] *= np.float32(2.0**-70)
+    w[:, i // 3] = w[:, i // 3 + 1] = rng.uniform(1, 2, o)
+    x[:, i // 3] = x[:, i // 3 + 1] = 0.0
+    x[0::3, i // 3], x[0::3, i // 3 + 1] = 1.5, -1.5
+    return x, w
+
+
+def serial_linear(x, w, denormal_inputs=True, denormal_products=True):
+    """oracle.linear's sums with denormal operands or products taken as 0."""
+    tiny = np.float32(2.0**-126)
+    if not denormal_inputs:
+        x, w = (np.where(np.abs(a) < tiny, np.float32(0), a) for a in (x, w))
+    s = np.zeros((x.shape[0], w.shape[0]), np.float32)
+    for k in range(x.shape[1]):
+        p = x[:, k, None] * w[None, :, k]
+        s = s + (p if denormal_products else np.where(np.abs(p) < tiny, np.float32(0), p))
+    return s
+
+
+def test_denormal_linear_case_tells_flushed_products():
+    """What test_gpu_linear_denormals_bit_exact rests on: products or operands
+    flushed to zero change the sums it expects in every kind of row."""
+    x, w = denormal_linear_case(9, 66, 64)
+    want = oracle.linear(x, w)
+    assert np.array_equal(serial_linear(x, w), want)
+    no_products = serial_linear(x, w, denormal_products=False) != want
+    no_operands = serial_linear(x, w, denormal_inputs=False) != want
+    dn = np.arange(64) % 4 == 3  # columns of denormal weights
+    for r in range(9):
+        assert no_products[r][dn if r % 3 == 2 else ~dn].mean() > 0.9, r
+    assert no_operands[2::3, dn].mean() > 0.9
+    assert (np.abs(want[0::3]) < 2.0**-120).all()  # the pair is gone
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,i,o", [
+    (1, 128, 40), (3, 64, 16),                           # 16 columns a wave
+    (6, 128, 2800), (16, 1024, 1025),                    # 64 columns a wave, one row each
+    (65, 260, 2049), (66, 65, 2111), (129, 4, 1100)])    # four rows a wave
+def test_gpu_linear_denormals_bit_exact(torch_dev, rows, i, o):
+    """Products are rounded as a multiplication rounds them, denormals included,
+    in every split (the four-row one takes them from the matrix cores)."""
+    torch, dev = torch_dev
+    x, w = denormal_linear_case(rows, i, o)
+    got = model.linear(torch.from_numpy(x).to(dev), torch.from_numpy(w).to(dev)).cpu().numpy()
+    want = oracle.linear(x, w)
+    assert (want != 0).mean() > 0.5
+    assert np.array_equal(got, want)
 
 
 @pytest.mark.gpu
