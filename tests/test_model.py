@@ -253,6 +253,18 @@ def test_gpu_linear_splits_bit_exact(torch_dev, rows, i, o, skew):
     assert np.array_equal(got, oracle.linear(x, w))
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,o", [(1, 2**26 + 17), (2, 2**28 + 65)])
+def test_gpu_linear_columns_past_one_grid_dimension(torch_dev, rows, o):
+    """Column counts whose groups need a second grid dimension (2^22 groups of
+    16 or 64): every column is there, the last group's too."""
+    torch, dev = torch_dev
+    w = torch.randn((o, 1), device=dev)
+    x = torch.tensor([[1.25], [-0.75]], device=dev)[:rows].contiguous()
+    got = model.linear(x, w)
+    assert torch.equal(got, x * w.view(1, o))
+
+
 def denormal_linear_case(rows, i, o):
     """x [rows, i], w [o, i] whose sums hold denormal terms only, once a pair
     +a, -a has cancelled in rows 0, 3, ...: products of normal numbers down to
@@ -368,7 +380,12 @@ def test_gpu_decoder_on_a_caller_stream(dev):
     (18, 768, 6, 2, "f32", True, True),       # ... whole pieces only
     (64, 136, 4, 4, "f32", True, True),       # 64 columns a wave, one row each
     (260, 192, 6, 2, "bf16", True, True),     # four rows a wave, an odd chunk at the end
-    (700, 72, 3, 1, "f32", False, False),     # ... without the norm
+    (700, 72, 3, 1, "f32", False, False),     # without the norm: 64 columns a wave, one row
+    (1030, 72, 3, 1, "f32", False, False),    # ... four rows
+    (1026, 64, 2, 1, "bf16", False, True),
+    (22, 257, 1, 1, "bf16", True, False),     # odd d_model: 64 columns a wave, one row
+    (86, 257, 1, 1, "f32", True, True),       # ... four rows
+    (67, 511, 7, 1, "bf16", True, True),
     (3, 33, 3, 1, "f32", True, True)])        # odd d_model: the scalar weight path
 def test_gpu_qkv_append_bit_exact(torch_dev, n, d, hq, hkv, dtype, ln, bias):
     """The fused LN1 -> q / k / v -> append launch equals the oracle's
@@ -587,6 +604,45 @@ def test_gpu_decoder_prompt_chunks(torch_dev, n_prompt, n_new, max_seq):
         got, lg = dec.generate(prompt, n_new, logits=True)
         assert got.tolist() == want.tolist()
         assert np.all(np.abs(lg - want_lg) <= np.maximum(1e-4, 1e-3 * np.abs(want_lg)))
+
+
+# d_model 2112, d_ff 1088: a pass of 64 prompt rows runs q / k / v, W_o and W_2
+# (residual, in place) and W_1 (GELU) with four rows a wave, a pass of one row
+# with one.
+WIDE_DECODER = dict(vocab=96, d_model=2112, n_heads=66, n_kv_heads=33, d_ff=1088, n_layers=1,
+                    max_seq=80)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,shape", [
+    (2, {}), (17, {}), (64, {}), (65, {}), (128, {}), (150, dict(max_seq=700)),
+    (64, WIDE_DECODER), (79, WIDE_DECODER)])
+def test_gpu_decoder_prompt_rows_have_the_bits_of_single_positions(torch_dev, n, shape):
+    """A position's logits do not depend on how many rows its pass had: n
+    positions generated one at a time, then given as one prompt."""
+    cfg = model.config(**shape)
+    params = model.init_params(cfg, seed=8, std=0.02)
+    dec = model.Decoder(cfg, params)
+    first = np.array([7], np.int32)
+    toks, lg = dec.generate(first, n, logits=True)  # position i from one row
+    prompt = np.concatenate([first, toks[:n - 1]])
+    tok, last = dec.generate(prompt, 1, logits=True)
+    assert tok[0] == toks[-1]
+    assert np.array_equal(last[0].view(np.int32), lg[-1].view(np.int32))
+
+
+@pytest.mark.gpu
+def test_gpu_wide_decoder_matches_oracle(torch_dev):
+    """Prompt passes with four rows a wave in every projection: tokens and
+    logits as the oracle's."""
+    cfg = model.config(**WIDE_DECODER)
+    params = model.init_params(cfg, seed=9, std=0.02)
+    prompt = np.random.default_rng(9).integers(0, cfg.vocab, 66).astype(np.int32)
+    want, want_lg = oracle.decoder_generate(oracle.decoder_config(**WIDE_DECODER), params, prompt,
+                                            3, logits=True)
+    got, lg = model.Decoder(cfg, params).generate(prompt, 3, logits=True)
+    assert got.tolist() == want.tolist()
+    assert np.all(np.abs(lg - want_lg) <= np.maximum(1e-4, 1e-3 * np.abs(want_lg)))
 
 
 @pytest.mark.gpu
