@@ -142,7 +142,7 @@ __global__ __launch_bounds__(64 * kMergeWaves) void decode_merge_kernel(
 }
 
 // Merge for calls with at most kMergeRowsMaxParts partitions per sequence
-// (max_context <= 8 partitions: configs[2] and most decode batches).  One
+// (max_context <= 8 partitions: 64 x U[512, 4096] and most decode batches).  One
 // wave per (sequence, query head), four per workgroup, no LDS and no
 // barrier: lane l holds float4 c = l % (D/4) of partition rows
 // p = l / (D/4) + RPW j, and the rows meet through cross-lane reductions.
@@ -239,11 +239,11 @@ int default_part(int dtype, int /*max_context*/) { return one_byte(dtype) ? kPQ 
 // per KV head, 1280 when the call holds work for at least 1,200 such
 // partitions over all KV heads (contexts taken as uniform up to cap), else
 // 768 when it holds work for 1,000 of those, else 640 when it holds work for
-// 800 partitions of 512, else 512 (the measurements above: configs[2] 768,
-// configs[3] and 256 x U[1, 8192] 1280; and, us per call at 512 / 640 /
+// 800 partitions of 512, else 512 (64 x U[512, 4096] 768, 8 x U[16384, 65536]
+// and 256 x U[1, 8192] 1280; and, us per call at 512 / 640 /
 // 768 over U[512, 4096] contexts, 32 layers back to back: 8 sequences x 8
-// KV heads 19.5 / 22.4 / 24.3, 64 x 1 (configs[2]'s share of one GPU of 8
-// by KV heads) 23.8 / 24.5 / 25.9, 16 x 8 33.4 / 38.9 / 35.9, 64 x 2 36.9 /
+// KV heads 19.5 / 22.4 / 24.3, 64 x 1 (one GPU's share of 8 KV heads split
+// over 8) 23.8 / 24.5 / 25.9, 16 x 8 33.4 / 38.9 / 35.9, 64 x 2 36.9 /
 // 41.4 / 40.7, 24 x 8 42.4 / 43.5 / 43.8, 32 x 8 56.4 / 56.5 / 55.7, 64 x 4
 // 60.8 / 58.9 / 64.6, 48 x 8 82.8 / 81.7 / 81.3).
 // The 512-token tier holds for fp32 pools and every head shape: 512 / 640

@@ -6,12 +6,14 @@
 // rounded as a product and then added (no fused multiply-add): the bits of the
 // reference's CPU loops.  So a sum cannot be split, and a term costs a
 // multiplication and an addition, and a wave issues one vector instruction
-// per 4 cycles: 8.4 cycles a term and row for one row per wave.  With four
-// rows per wave the multiplications run on the matrix cores instead:
+// per 4 cycles: of a wave of one row's 15 cycles a term (SQ counters, n = 4,096)
+// it issues in 9.  With four rows per wave the multiplications run on the
+// matrix cores instead:
 // v_mfma_f32_4x4x1_16b_f32 with C = 0 gives 256 products fma(x, w, 0), each
 // rounded once (checked bit for bit on gfx950, denormals included; the sign
 // of a zero product may differ, which no sum that starts at +0 shows), and
-// the vector unit only adds: 27 cycles a term for the four rows.
+// the vector unit only adds: 37 cycles a term for the four rows, 21 of them
+// issuing.
 #include <cmath>
 
 #include "model_ops.hpp"
@@ -276,8 +278,8 @@ __device__ __forceinline__ float row_bcast(float x) {
 // four rows (lane 4 j + i: row i, features 4 j .. + 3), and cbsz = 4 /
 // abid = j hand the lanes of block j to all 16 blocks -- and result register e
 // is row e of every column.  A group's MFMAs are issued before the additions
-// of the group before, so no addition waits for its product: grouped like this
-// four rows cost 33 cycles a feature, alternating one by one 41.
+// of the group before, so no addition waits for its product (37 cycles a
+// feature and four rows; alternating the two one by one is a quarter slower).
 // RW = 1: lane j of each 16 holds features 4 j .. + 3 of the row and
 // row_newbcast hands one to the multiplication.
 // Weights pass through LDS, a chunk of 64 features in each of three buffers:

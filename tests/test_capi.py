@@ -92,8 +92,8 @@ def test_workspace_size():
     # the one-call pick by shape: bf16, head_dim 128, <= 4 query heads per KV
     # head; 1280 with work for >= 1200 such partitions, 768 with work for >=
     # 1000 of those, 640 with work for >= 800 partitions of 512, else 512
-    # (configs[2]: 768; configs[3] and 256 x 8192: 1280; configs[2]'s share
-    # of one GPU of 8: 512; above the 512 tier, 8 heads per KV head, head_dim
+    # (64 x 4096: 768; 8 x 65536 and 256 x 8192: 1280; one GPU's share of 64 x
+    # 4096 over 8: 512; above the 512 tier, 8 heads per KV head, head_dim
     # 64, fp32 and 1-byte pools: 640)
     F = L.rkv_decode_partition_size_for
     assert F(0, 64, 32, 8, 128, RKV_BF16, 4096) == 768
