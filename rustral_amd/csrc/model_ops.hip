@@ -406,11 +406,14 @@ extern "C" int rkv_argmax(int32_t* out, const float* x, int rows, int n, void* s
   if (rows == 0) return RKV_OK;
   if (!out || !x) return fail(RKV_ERR_INVALID_ARG, "rkv_argmax: null pointer argument");
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  // Four waves cut a long row's chain of loads (us, four / one: 1 row of 4,096
-  // 3.9 / 5.5, of 32,000 9.4 / 25.6); up to 1,024 columns they only cost
+  // Four waves cut a long row's chain of loads (us, four / one: 1 row of 2,000
+  // 3.9 / 4.4, of 32,000 9.4 / 25.6); up to 1,024 columns they only cost
   // workgroups (1 x 1,000 3.6 / 3.7; 4,096 x 256 6.7 / 4.3; 65,536 x 100 51 /
-  // 19).  2^24 rows of four waves would be 2^32 threads, at which a grid wraps.
-  if (n <= 1024 || rows >= 1 << 24)
+  // 19), and up to 2,048 where the rows fill the chip (2,048 x 2,000 5.8 / 7.2,
+  // 4,096 x 2,000 10.1 / 8.4, 65,536 x 2,000 139 / 98; 4,096 columns alike or
+  // ahead with four).  2^24 rows of four waves would be 2^32 threads, at which a
+  // grid wraps.
+  if (n <= 1024 || (n <= 2048 && rows >= 4096) || rows >= 1 << 24)
     argmax_kernel<1, false><<<(unsigned)rows, 64, 0, s>>>(out, x, n, EmbedTail{});
   else
     argmax_kernel<4, false><<<(unsigned)rows, 256, 0, s>>>(out, x, n, EmbedTail{});

@@ -463,7 +463,7 @@ def test_gpu_argmax_matches_reference_rule(torch_dev):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 1024, 1025, 2500])
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 257, 1024, 1025, 2048, 2049])
 def test_gpu_argmax_row_lengths(torch_dev, n):
     """Rows on both sides of the one-wave / four-wave line and at the waves'
     edges: random, tied, all -inf and NaN at either end."""
@@ -477,6 +477,9 @@ def test_gpu_argmax_row_lengths(torch_dev, n):
     x = np.stack(rows).astype(np.float32)
     got = model.argmax(torch.from_numpy(x).to(dev)).cpu().numpy()
     assert got.tolist() == [oracle.argmax(r) for r in x]
+    many = np.concatenate([x] * (4096 // len(x) + 1))  # one wave up to 2,048 columns
+    assert (model.argmax(torch.from_numpy(many).to(dev)).cpu().numpy()
+            == np.tile(got, 4096 // len(x) + 1)).all()
 
 
 @pytest.mark.gpu
